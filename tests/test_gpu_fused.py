@@ -39,6 +39,49 @@ def test_ssd_scan(dev, dtype, disc, P, N):
     assert_close(hl, h_ref, TOL[dtype], "ssd h_last")
 
 
+@pytest.mark.parametrize("dtype,B,L,H,P,N,chunk,form", [
+    (torch.float32, 1, 1, 1, 16, 8, 256, "plain"),        # one step, half a block of columns
+    (torch.float32, 2, 15, 3, 31, 16, 256, "plain"),      # no vector access: P odd
+    (torch.float32, 1, 17, 2, 64, 64, 256, "slow"),
+    (torch.float32, 3, 4001, 5, 64, 64, 256, "slow"),     # segments, no decay reaches zero
+    (torch.float32, 2, 3000, 4, 40, 32, 64, "fast"),      # segments, early stops
+    (torch.float32, 2, 700, 3, 24, 16, 256, "shifted"),   # vector width but misaligned base
+    (torch.float16, 2, 1500, 3, 64, 32, 256, "slow"),
+    (torch.float16, 1, 90, 2, 36, 64, 256, "plain"),      # P no multiple of a 16-byte access
+    (torch.bfloat16, 2, 2000, 3, 32, 16, 128, "slow"),
+    (torch.bfloat16, 1, 130, 2, 64, 8, 256, "plain"),
+    (torch.float32, 1, 300, 2, 48, 32, 256, "inf"),
+])
+def test_ssd_scan_walk(dev, dtype, B, L, H, P, N, chunk, form):
+    """The fp32-product walk (every form the bf16 kernels do not take) at the
+    edges of its blocks, channel and column tiles, vector accesses and
+    segments.  fp32 results must be within 2e-6 of float64 (normwise): sums
+    over at most a few hundred live steps at 6e-8 each, in random order.
+    "inf": an infinite input must leave every earlier step as it was."""
+    from tssm import ssd_scan_forward
+    d = _ssd_inputs(dev, B, L, H, P, N, dtype, seed=L + P + N, heavy=form == "fast")
+    if form == "slow":
+        d["dt"] = d["dt"] * 0.002
+    if form == "shifted":
+        for k in ("x", "B"):
+            t = d[k]
+            flat = torch.empty(t.numel() + 1, device=dev, dtype=dtype)
+            d[k] = flat[1:].view(t.shape).copy_(t)
+    h0 = torch.randn(B, H, P, N, device=dev)
+    args = (d["dt"], d["A_log"], d["B"], d["C"], d["D"])
+    y, hl = ssd_scan_forward(d["x"], *args, h0=h0, chunk=chunk, return_state=True)
+    y_ref, h_ref = O.ssd_scan(d["x"], *args, h0=np64(h0))
+    tol = 2e-6 if dtype == torch.float32 else TOL[dtype]
+    assert_close(y, y_ref, tol, f"walk y {dtype} {form}")
+    assert_close(hl, h_ref, 2e-6, "walk h_last")
+    if form == "inf":
+        x = d["x"].clone()
+        x[:, 151, :, 7] = float("inf")
+        bad = ssd_scan_forward(x, *args, h0=h0, chunk=chunk)
+        torch.testing.assert_close(bad[:, :151], y[:, :151], rtol=0, atol=0)
+        assert not bool(torch.isfinite(bad[:, 151, :, 7]).any())
+
+
 @pytest.mark.parametrize("L", [100, 256, 513, 2600])
 @pytest.mark.parametrize("disc", ["zoh", "euler"])
 @pytest.mark.parametrize("with_d", [False, True])

@@ -349,6 +349,8 @@ inline bool aligned(const void* p, uintptr_t a) {
   return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
 }
 
+inline int64_t cdiv64(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 }  // namespace tssm

@@ -288,7 +288,6 @@ __global__ __launch_bounds__(64 * kRedWaves) void zoh_bwd_pass2_kernel(
   }
 }
 
-inline int64_t cdiv64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 }  // namespace tssm
 

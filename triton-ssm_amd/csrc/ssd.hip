@@ -6,20 +6,11 @@
 // ssm_scan.py:5-10 with the discretization of discretize_kernel.py:44-54 and
 // one decay per head.
 //
-// ssd_scan: three passes (chunk states, state passing, chunk outputs).  With
-// few (batch, head) rows and very long sequences a single pass would keep
-// hundreds of chunks of one row in flight, each look-back hop moving a whole
-// P x N state; the passes instead re-read x, B and dt once.
-//   pass 1 ssd_state_kernel: one wave per (row, chunk of TC steps), lane = p
-//     with its N states in registers; writes the chunk's decay product and
-//     local end state (from zero).
-//   pass 2 ssd_pass_kernel: per state entry, a segmented scan over chunks
-//     gives every chunk's entry state (and the final state).
-//   pass 3 ssd_out_kernel: one wave per chunk rescans from its entry state and
-//     writes y.
-//   Both scans use the rescaled state h_t = P_t g_t (P_t = decay product since
-//   the chunk start), so a step costs one FMA per state for the update; g is
-//   folded back into h whenever P_t would drop below 2^-64.
+// ssd_scan, bf16 with P = 64, N = 16 and 256-step chunks: one launch
+// (ssd_fused_wave_kernel) or three tile passes on the bf16 matrix cores (chunk
+// states, ssd_pass_kernel passing the states, chunk outputs).  bf16 with
+// N = 64 takes ssd_n64.hip, everything else the fp32-product walk of
+// ssd_walk.hip.
 // ssd_stream_step_kernel: one streaming step with the state [S,H,P,N] fp32
 //   resident in HBM, updated in place; one workgroup per (stream, head).
 #include "common.h"
@@ -28,187 +19,6 @@
 #include "ssd_dev.h"
 
 namespace tssm {
-
-constexpr float kRescaleFloor = 5.421010862427522e-20f;  // 2^-64
-constexpr int kSsdSub = 16;  // steps staged per sub-block
-
-// One step of the rescaled recurrence h = Pt g:  h_t = ab h_{t-1} + xs B_t.
-// When Pt ab would fall below 2^-64 the factor is folded into g (the branch is
-// uniform: Pt and ab are the same on every lane of the wave).
-template <int N>
-__device__ inline void rescaled_step(float* g, float& Pt, float ab, float xs, const float* bv) {
-  // Pt and ab hold the same value on every lane; reading the product through
-  // lane 0 makes the fold decision a scalar branch.
-  const float Pn = __builtin_bit_cast(
-      float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, Pt * ab)));
-  if (Pn < kRescaleFloor) {
-#pragma unroll
-    for (int n = 0; n < N; ++n) g[n] = __builtin_fmaf(xs, bv[n], g[n] * Pn);
-    Pt = 1.0f;
-  } else {
-    const float xr = xs * __builtin_amdgcn_rcpf(Pn);
-#pragma unroll
-    for (int n = 0; n < N; ++n) g[n] = __builtin_fmaf(xr, bv[n], g[n]);
-    Pt = Pn;
-  }
-}
-
-// Registers of one sub-block of kSsdSub steps: x of the lane's channel and
-// the B (and, for the outputs, C) rows, spread over the wave.  Every load of
-// a sub-block is issued before the first is used: clamped addresses (steps
-// past L re-read step L-1) and selects at the LDS store, no branch around a
-// load (the compiler would wait for a load inside a branch on its own).
-//
-// With kSsdPipe<N> the loads of sub-block k+1 (and the dt of the next 64-step
-// group) are issued before sub-block k is computed from LDS, so they are in
-// flight during its steps.  That holds one more sub-block in registers:
-// fp32 at L=65536 H=8 P=64: N=16 195.98 -> 178.13 us (state 76 -> 109,
-// output 87 -> 127 VGPRs), N=32 267.1 -> 253.2 us; at N=64 the output pass
-// drops to one wave per SIMD and the passes slow 432.4 -> 585.7 us, so N=64
-// loads each sub-block just before it is used.
-template <int N>
-constexpr bool kSsdPipe = N <= 32;
-
-template <int N, bool WITH_C>
-struct SsdSub {
-  static constexpr int K = (kSsdSub * N + 63) / 64;
-  float x[kSsdSub], b[K], c[WITH_C ? K : 1];
-};
-
-template <typename T, int N, bool WITH_C>
-__device__ inline void sub_load(SsdSub<N, WITH_C>& r, const T* __restrict__ xp, int64_t sx_l,
-                                const T* __restrict__ Bp, int64_t sB_l, const T* __restrict__ Cp,
-                                int64_t sC_l, int64_t ts, int64_t L, int lane) {
-#pragma unroll
-  for (int i = 0; i < kSsdSub; ++i) {
-    const int64_t t = ts + i;
-    r.x[i] = ldf(xp + (t < L ? t : L - 1) * sx_l);
-  }
-#pragma unroll
-  for (int q = 0; q < SsdSub<N, WITH_C>::K; ++q) {
-    const int k = lane + 64 * q;
-    const int kc = k < kSsdSub * N ? k : 0;
-    const int i = kc / N, n = kc - (kc / N) * N;
-    const int64_t t = ts + i < L ? ts + i : L - 1;
-    r.b[q] = ldf(Bp + t * sB_l + n);
-    if constexpr (WITH_C) r.c[q] = ldf(Cp + t * sC_l + n);
-  }
-}
-
-template <int N, bool WITH_C>
-__device__ inline void sub_store(const SsdSub<N, WITH_C>& r, int64_t ts, int64_t L, bool act,
-                                 float* s_x, float* s_B, float* s_C, int lane) {
-#pragma unroll
-  for (int i = 0; i < kSsdSub; ++i) s_x[i * 64 + lane] = (act && ts + i < L) ? r.x[i] : 0.0f;
-#pragma unroll
-  for (int q = 0; q < SsdSub<N, WITH_C>::K; ++q) {
-    const int k = lane + 64 * q;
-    if (k < kSsdSub * N) {
-      const bool in = ts + k / N < L;
-      s_B[k] = in ? r.b[q] : 0.0f;
-      if constexpr (WITH_C) s_C[k] = in ? r.c[q] : 0.0f;
-    }
-  }
-}
-
-// dt of step t0 + lane (clamped address; steps at or past L are zeroed by
-// step_scalars_of).
-__device__ inline float dt_ahead(const float* dtp, int64_t sdt_l, int64_t t0, int64_t L,
-                                 int lane) {
-  const int64_t t = t0 + lane;
-  return dtp[(t < L ? t : L - 1) * sdt_l];
-}
-
-// Per-step decay and input coefficient for steps [t0, t0+64) of one head,
-// computed by lane i for step t0+i from its dt and shared through LDS.  Steps
-// at or past L get dt = 0, i.e. decay 1 and coefficient 0, so they leave the
-// state alone.
-template <int DISC>
-__device__ inline void step_scalars_of(float dl, int64_t t0, int64_t L, float a2, float* s_ab,
-                                       float* s_cf, int lane) {
-  const float d = t0 + lane < L ? dl : 0.0f;
-  const float arg = d * a2;
-  const float ab = exp2_fast(arg);
-  s_ab[lane] = ab;
-  s_cf[lane] = (DISC == TSSM_DISC_ZOH) ? phi1_from_exp(arg * 0.6931471805599453f, ab) * d : d;
-}
-
-// Pass 1 of the generic passes: the chunk's end state from a zero state,
-// walked last step first, X += R_s coef_s x_s B_s with R_s the decay from
-// step s+1 to the chunk end (a running product of the per-step decays), and
-// the chunk's decay product R.  Once R has underflowed to exactly zero every
-// earlier step adds an exact zero: the walk stops there (uniform: R depends
-// only on the head's dt), and the decay product is zero.
-template <typename T, int DISC, int N>
-__global__ __launch_bounds__(64) void ssd_state_kernel(SsdArgs a) {
-  __shared__ float s_ab[64], s_cf[64];
-  __shared__ __align__(16) float s_B[kSsdSub * N];
-  __shared__ float s_x[kSsdSub * 64];
-  const int lane = threadIdx.x;
-  const int P = (int)a.P;
-  const bool act = lane < P;
-  const uint32_t row = blockIdx.x / a.nchunks;
-  const uint32_t c = blockIdx.x - row * a.nchunks;
-  const uint32_t b = row / a.H, h = row - (row / a.H) * a.H;
-  const float a2 = -expf(a.A_log[h]) * kLog2e;
-  const int64_t tbeg = (int64_t)c * a.tc;
-  const int64_t tend = tbeg + a.tc < a.L ? tbeg + a.tc : a.L;
-  const float* dtp = a.dt + b * a.sdt_b + h * a.sdt_h;
-  const T* xp = reinterpret_cast<const T*>(a.x) + b * a.sx_b + h * a.sx_h + (act ? lane : 0);
-  const T* Bp = reinterpret_cast<const T*>(a.B) + b * a.sB_b + h * a.sB_h;
-  float g[N];
-#pragma unroll
-  for (int n = 0; n < N; ++n) g[n] = 0.0f;
-  float R = 1.0f;
-  constexpr bool PIPE = kSsdPipe<N>;
-  // sub-blocks of kSsdSub steps (a.tc is a multiple of 64), walked from the
-  // last; each 64-step group's step scalars are formed on entering it
-  const int64_t nsb = (tend - tbeg + kSsdSub - 1) / kSsdSub;
-  auto group_t0 = [&](int64_t k) { return tbeg + (k * kSsdSub) / 64 * 64; };
-  SsdSub<N, false> nxt;
-  float dnext = 0.0f;
-  if constexpr (PIPE) {
-    sub_load<T, N, false>(nxt, xp, a.sx_l, Bp, a.sB_l, Bp, 0, tbeg + (nsb - 1) * kSsdSub, a.L,
-                          lane);
-    dnext = dt_ahead(dtp, a.sdt_l, group_t0(nsb - 1), a.L, lane);
-  }
-  for (int64_t k = nsb - 1; k >= 0; --k) {
-    const int64_t ts = tbeg + k * kSsdSub;
-    const int64_t t0 = group_t0(k);
-    const int j = (int)(ts - t0);
-    if (k == nsb - 1 || j + kSsdSub == 64) {  // entering a group from its end
-      if constexpr (PIPE) {
-        step_scalars_of<DISC>(dnext, t0, a.L, a2, s_ab, s_cf, lane);
-        dnext = dt_ahead(dtp, a.sdt_l, t0 > tbeg ? t0 - 64 : tbeg, a.L, lane);
-      } else {
-        step_scalars_of<DISC>(dt_ahead(dtp, a.sdt_l, t0, a.L, lane), t0, a.L, a2, s_ab, s_cf,
-                              lane);
-      }
-    }
-    if constexpr (!PIPE) sub_load<T, N, false>(nxt, xp, a.sx_l, Bp, a.sB_l, Bp, 0, ts, a.L, lane);
-    sub_store<N, false>(nxt, ts, a.L, act, s_x, s_B, s_B, lane);
-    __syncthreads();
-    if constexpr (PIPE)
-      sub_load<T, N, false>(nxt, xp, a.sx_l, Bp, a.sB_l, Bp, 0, k > 0 ? ts - kSsdSub : ts, a.L,
-                            lane);
-#pragma unroll 2
-    for (int i = kSsdSub - 1; i >= 0; --i) {
-      const float w = R * (s_cf[j + i] * s_x[i * 64 + lane]);
-#pragma unroll
-      for (int n = 0; n < N; ++n) g[n] = __builtin_fmaf(w, s_B[i * N + n], g[n]);
-      R *= s_ab[j + i];
-    }
-    __syncthreads();
-    if (R == 0.0f) break;  // uniform: the earlier steps add exact zeros
-  }
-  const int64_t PN = (int64_t)P * N;
-  if (act) {
-    float* out = a.chunkX + ((int64_t)row * a.nchunks + c) * PN + (int64_t)lane * N;
-#pragma unroll
-    for (int n = 0; n < N; ++n) out[n] = g[n];
-  }
-  if (lane == 0) a.chunkA[(int64_t)row * a.nchunks + c] = R;
-}
 
 // Pass 2: thread (entry e, segment sg) of a 1024-thread workgroup covering 32
 // consecutive state entries of one row and 32 segments of its chunks.  A
@@ -305,77 +115,6 @@ __global__ __launch_bounds__(1024) void ssd_pass_kernel(SsdArgs a, int64_t PN) {
     }
   }
   if (act && a.h_last && sg == kPassSegs - 1) a.h_last[row * PN + e] = S;
-}
-
-template <typename T, int DISC, int N, bool HAS_D>
-__global__ __launch_bounds__(64) void ssd_out_kernel(SsdArgs a) {
-  __shared__ float s_ab[64], s_cf[64];
-  __shared__ __align__(16) float s_B[kSsdSub * N];
-  __shared__ __align__(16) float s_C[kSsdSub * N];
-  __shared__ float s_x[kSsdSub * 64];
-  const int lane = threadIdx.x;
-  const int P = (int)a.P;
-  const bool act = lane < P;
-  const uint32_t row = blockIdx.x / a.nchunks;
-  const uint32_t c = blockIdx.x - row * a.nchunks;
-  const uint32_t b = row / a.H, h = row - (row / a.H) * a.H;
-  const float a2 = -expf(a.A_log[h]) * kLog2e;
-  const int64_t tbeg = (int64_t)c * a.tc;
-  const int64_t tend = tbeg + a.tc < a.L ? tbeg + a.tc : a.L;
-  const float* dtp = a.dt + b * a.sdt_b + h * a.sdt_h;
-  const T* xp = reinterpret_cast<const T*>(a.x) + b * a.sx_b + h * a.sx_h + (act ? lane : 0);
-  const T* Bp = reinterpret_cast<const T*>(a.B) + b * a.sB_b + h * a.sB_h;
-  const T* Cp = reinterpret_cast<const T*>(a.C) + b * a.sC_b + h * a.sC_h;
-  T* yp = reinterpret_cast<T*>(a.y) + b * a.sy_b + h * a.sy_h + (act ? lane : 0);
-  const int64_t PN = (int64_t)P * N;
-  float g[N];
-  {
-    const float* en = a.entry + ((int64_t)row * a.nchunks + c) * PN + (int64_t)(act ? lane : 0) * N;
-#pragma unroll
-    for (int n = 0; n < N; ++n) g[n] = act ? en[n] : 0.0f;
-  }
-  const float dv = (HAS_D && act) ? a.D[h * P + lane] : 0.0f;
-  float Pt = 1.0f;
-  constexpr bool PIPE = kSsdPipe<N>;
-  SsdSub<N, true> nxt;
-  float dnext = 0.0f;
-  if constexpr (PIPE) {
-    sub_load<T, N, true>(nxt, xp, a.sx_l, Bp, a.sB_l, Cp, a.sC_l, tbeg, a.L, lane);
-    dnext = dt_ahead(dtp, a.sdt_l, tbeg, a.L, lane);
-  }
-  for (int64_t t0 = tbeg; t0 < tend; t0 += 64) {
-    if constexpr (PIPE) {
-      step_scalars_of<DISC>(dnext, t0, a.L, a2, s_ab, s_cf, lane);
-      dnext = dt_ahead(dtp, a.sdt_l, t0 + 64, a.L, lane);
-    } else {
-      step_scalars_of<DISC>(dt_ahead(dtp, a.sdt_l, t0, a.L, lane), t0, a.L, a2, s_ab, s_cf, lane);
-    }
-    for (int j = 0; j < 64 && t0 + j < tend; j += kSsdSub) {
-      const int64_t ts = t0 + j;
-      if constexpr (!PIPE)
-        sub_load<T, N, true>(nxt, xp, a.sx_l, Bp, a.sB_l, Cp, a.sC_l, ts, a.L, lane);
-      sub_store<N, true>(nxt, ts, a.L, act, s_x, s_B, s_C, lane);
-      __syncthreads();
-      if constexpr (PIPE)
-        sub_load<T, N, true>(nxt, xp, a.sx_l, Bp, a.sB_l, Cp, a.sC_l, ts + kSsdSub, a.L, lane);
-      const int m = a.L - ts < kSsdSub ? (int)(a.L - ts) : kSsdSub;
-#pragma unroll 2
-      for (int i = 0; i < kSsdSub; ++i) {
-        const float xv = s_x[i * 64 + lane];
-        float bv[N];
-#pragma unroll
-        for (int n = 0; n < N; ++n) bv[n] = s_B[i * N + n];
-        rescaled_step<N>(g, Pt, s_ab[j + i], s_cf[j + i] * xv, bv);
-        float acc = 0.0f;
-#pragma unroll
-        for (int n = 0; n < N; ++n) acc = __builtin_fmaf(s_C[i * N + n], g[n], acc);
-        acc *= Pt;
-        if (HAS_D) acc = __builtin_fmaf(dv, xv, acc);
-        if (act && i < m) stf(yp + (ts + i) * a.sy_l, acc);
-      }
-      __syncthreads();
-    }
-  }
 }
 
 // ---------------------------------------------------------------- streaming step
@@ -1144,39 +883,6 @@ int launch_ssd_mfma(bool has_d, int64_t rows, int64_t nchunks, int64_t PN, hipSt
 }
 
 
-inline int64_t cdiv64(int64_t x, int64_t y) { return (x + y - 1) / y; }
-
-template <typename T, int DISC, int N, bool HAS_D>
-int launch_ssd_passes(int64_t rows, int64_t nchunks, int64_t PN, hipStream_t s, const SsdArgs& a) {
-  const dim3 tiles((unsigned)(rows * nchunks));
-  hipLaunchKernelGGL((ssd_state_kernel<T, DISC, N>), tiles, dim3(64), 0, s, a);
-  const int64_t nblk = (PN + kPassEntries - 1) / kPassEntries;
-  hipLaunchKernelGGL(ssd_pass_kernel, dim3((unsigned)(rows * nblk)), dim3(kPassEntries * kPassSegs),
-                     0, s, a, PN);
-  hipLaunchKernelGGL((ssd_out_kernel<T, DISC, N, HAS_D>), tiles, dim3(64), 0, s, a);
-  return launch_status();
-}
-
-template <typename T, int DISC, bool HAS_D>
-int launch_ssd_n(int N, int64_t rows, int64_t nchunks, int64_t PN, hipStream_t s, const SsdArgs& a) {
-  switch (N) {
-    case 8: return launch_ssd_passes<T, DISC, 8, HAS_D>(rows, nchunks, PN, s, a);
-    case 16: return launch_ssd_passes<T, DISC, 16, HAS_D>(rows, nchunks, PN, s, a);
-    case 32: return launch_ssd_passes<T, DISC, 32, HAS_D>(rows, nchunks, PN, s, a);
-    case 64: return launch_ssd_passes<T, DISC, 64, HAS_D>(rows, nchunks, PN, s, a);
-    default: return TSSM_ERR_UNSUPPORTED;
-  }
-}
-
-template <typename T>
-int launch_ssd_t(int disc, bool has_d, int N, int64_t rows, int64_t nchunks, int64_t PN,
-                 hipStream_t s, const SsdArgs& a) {
-  if (disc == TSSM_DISC_ZOH)
-    return has_d ? launch_ssd_n<T, TSSM_DISC_ZOH, true>(N, rows, nchunks, PN, s, a)
-                 : launch_ssd_n<T, TSSM_DISC_ZOH, false>(N, rows, nchunks, PN, s, a);
-  return has_d ? launch_ssd_n<T, TSSM_DISC_EULER, true>(N, rows, nchunks, PN, s, a)
-               : launch_ssd_n<T, TSSM_DISC_EULER, false>(N, rows, nchunks, PN, s, a);
-}
 
 // Steps per chunk: the `chunk` hint rounded to a multiple of 64 in [64, 1024].
 inline int64_t ssd_tc(int64_t chunk) {
@@ -1264,11 +970,7 @@ extern "C" int tssm_ssd_scan(int dtype, int disc, const void* x, const float* dt
       sC_b % 8 == 0 && sy_l % 4 == 0 && sy_h % 4 == 0 && sy_b % 4 == 0 &&
       rows * (P / kSqP) < (int64_t)INT32_MAX)
     return launch_ssd_seq_any(disc, has_d, rows, P, s, a);
-  switch (dtype) {
-    case TSSM_BF16: return launch_ssd_t<bf16_t>(disc, has_d, (int)N, rows, nchunks, PN, s, a);
-    case TSSM_F16: return launch_ssd_t<f16_t>(disc, has_d, (int)N, rows, nchunks, PN, s, a);
-    default: return launch_ssd_t<float>(disc, has_d, (int)N, rows, nchunks, PN, s, a);
-  }
+  return launch_ssd_walk(dtype, disc, (int)N, s, a);
 }
 
 namespace tssm {

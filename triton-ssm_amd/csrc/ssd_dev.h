@@ -88,4 +88,8 @@ constexpr int kSqP = 16;   // channels per product tile (a workgroup takes 1 or 
 int launch_ssd_seq_any(int disc, bool has_d, int64_t rows, int64_t P, hipStream_t s,
                        const SsdArgs& a);
 
+// Every other operand form, with fp32 matrix products (ssd_walk.hip); the
+// workspace is a.chunkX .. a.chunkA + rows x nchunks.
+int launch_ssd_walk(int dtype, int disc, int N, hipStream_t s, const SsdArgs& a);
+
 }  // namespace tssm
