@@ -101,4 +101,6 @@ def check(code: int, what: str) -> None:
 
 def call(name: str, *args) -> None:
     """Call an int-returning entry point and raise on a nonzero status."""
-    check(getattr(lib(), name)(*args), name)
+    code = getattr(_lib or lib(), name)(*args)
+    if code != 0:
+        check(code, name)

@@ -27,6 +27,14 @@ def _inner_unit(t: torch.Tensor, what: str) -> None:
         raise ValueError(f"{what}: innermost dimension must be contiguous")
 
 
+def _rows(t: torch.Tensor, what: str) -> tuple:
+    """Strides of every dimension but the innermost, which must be contiguous."""
+    s = t.stride()
+    if s[-1] != 1:
+        raise ValueError(f"{what}: innermost dimension must be contiguous")
+    return s[:-1]
+
+
 def multihead_ssm_forward(u, A_log, B, C, dt, D=None, *, chunk=128, disc="euler", h0=None,
                           return_state=False, out=None):
     """Fused DIAG multihead selective scan.
@@ -62,8 +70,7 @@ def multihead_ssm_forward(u, A_log, B, C, dt, D=None, *, chunk=128, disc="euler"
         raise ValueError(f"A_log must be [nh] or [nh, hd], got {tuple(A_log.shape)}")
     A_log = as_f32(A_log, "A_log").contiguous()
     dt = as_f32(dt, "dt")
-    for t, w in ((u, "u"), (B, "B"), (C, "C")):
-        _inner_unit(t, w)
+    su, sB, sC = _rows(u, "u"), _rows(B, "B"), _rows(C, "C")
     if D is not None:
         need_gpu(D, "D")
         if D.numel() != nh * hd:
@@ -78,7 +85,7 @@ def multihead_ssm_forward(u, A_log, B, C, dt, D=None, *, chunk=128, disc="euler"
     need_gpu(y, "out")
     if y.shape != u.shape or y.dtype != u.dtype:
         raise ValueError("out must match u in shape and dtype")
-    _inner_unit(y, "out")
+    sy = _rows(y, "out")
     h_last = torch.empty(Bsz, nh, hd, device=u.device, dtype=torch.float32) if return_state else None
 
     L_ = _lib.lib()
@@ -89,10 +96,8 @@ def multihead_ssm_forward(u, A_log, B, C, dt, D=None, *, chunk=128, disc="euler"
     ws = workspace.get(u.device, stream, nbytes)
     _lib.call("tssm_mh_scan_fused", code, _disc_code(disc), u.data_ptr(), A_log.data_ptr(),
               B.data_ptr(), C.data_ptr(), dt.data_ptr(), ptr(D), ptr(h0), y.data_ptr(),
-              ptr(h_last), Bsz, L, nh, hd, int(a_per_head), u.stride(0), u.stride(1),
-              B.stride(0), B.stride(1), B.stride(2), C.stride(0), C.stride(1), C.stride(2),
-              dt.stride(0), dt.stride(1), dt.stride(2), y.stride(0), y.stride(1), int(chunk),
-              ws.data_ptr(), ws.numel(), stream)
+              ptr(h_last), Bsz, L, nh, hd, int(a_per_head), *su, *sB, *sC, *dt.stride(), *sy,
+              int(chunk), ws.data_ptr(), ws.numel(), stream)
     return (y, h_last) if return_state else y
 
 
@@ -133,8 +138,7 @@ def ssd_scan_forward(x, dt, A_log, B, C, D=None, *, chunk=256, disc="zoh", h0=No
     if B.dtype != x.dtype or C.dtype != x.dtype:
         raise TypeError("x, B and C must share one dtype")
     code = dcode(x, "x")
-    for t, w in ((x, "x"), (B, "B"), (C, "C")):
-        _inner_unit(t, w)
+    sx, sB, sC = _rows(x, "x"), _rows(B, "B"), _rows(C, "C")
     A_log = as_f32(A_log, "A_log").contiguous()
     dt = as_f32(dt, "dt")
     if D is not None:
@@ -151,13 +155,14 @@ def ssd_scan_forward(x, dt, A_log, B, C, D=None, *, chunk=256, disc="zoh", h0=No
     need_gpu(y, "out")
     if y.shape != x.shape or y.dtype != x.dtype:
         raise ValueError("out must match x in shape and dtype")
-    _inner_unit(y, "out")
+    sy = _rows(y, "out")
     h_last = torch.empty(Bsz, H, P, N, device=x.device, dtype=torch.float32) if return_state else None
     L_ = _lib.lib()
     args = (x.data_ptr(), dt.data_ptr(), A_log.data_ptr(), B.data_ptr(), C.data_ptr(), ptr(D),
-            ptr(h0), y.data_ptr(), ptr(h_last), Bsz, L, H, P, N, *x.stride()[:3], *dt.stride(),
-            *B.stride()[:3], *C.stride()[:3], *y.stride()[:3], int(chunk))
-    if fused and L_.tssm_ssd_scan_fused_supported(code, *args):
+            ptr(h0), y.data_ptr(), ptr(h_last), Bsz, L, H, P, N, *sx, *dt.stride(), *sB, *sC, *sy,
+            int(chunk))
+    # (the one-launch form exists for bf16 and N = 16 only: no need to ask for others)
+    if fused and N == 16 and code == _lib.BF16 and L_.tssm_ssd_scan_fused_supported(code, *args):
         # one launch with a decoupled look-back: a look-back workspace
         ws, stream = _ws(L_.tssm_ssd_scan_fused_workspace_bytes(Bsz, L, H, P, N, int(chunk)), x,
                          "ssd_scan")
@@ -388,8 +393,7 @@ def selective_scan_forward(x, dt, A_log, B=None, C=None, D=None, *, chunk=128, d
     if B.dtype != x.dtype or C.dtype != x.dtype:
         raise TypeError("x, B and C must share one dtype")
     code = dcode(x, "x")
-    for t, w in ((x, "x"), (B, "B"), (C, "C")):
-        _inner_unit(t, w)
+    sx, sB, sC = _rows(x, "x"), _rows(B, "B"), _rows(C, "C")
     dt = as_f32(dt, "dt")
     proj = None
     if dt_proj is not None:
@@ -432,7 +436,7 @@ def selective_scan_forward(x, dt, A_log, B=None, C=None, D=None, *, chunk=128, d
     need_gpu(y, "out")
     if y.shape != x.shape or y.dtype != x.dtype:
         raise ValueError("out must match x in shape and dtype")
-    _inner_unit(y, "out")
+    sy = _rows(y, "out")
     h_last = torch.empty(Bsz, Dc, N, device=x.device, dtype=torch.float32) if return_state else None
     L_ = _lib.lib()
     # the three-pass path writes raw fp32 chunk states (and the produced dt)
@@ -455,16 +459,13 @@ def selective_scan_forward(x, dt, A_log, B=None, C=None, D=None, *, chunk=128, d
         _lib.call("tssm_selective_scan_dtproj", code, _disc_code(disc), x.data_ptr(),
                   dt.data_ptr(), W.data_ptr(), bias.data_ptr(), dt_min, dt_max,
                   A_log.data_ptr(), B.data_ptr(), C.data_ptr(), ptr(D), ptr(h0), y.data_ptr(),
-                  ptr(h_last), Bsz, L, Dc, N, rank, x.stride(0), x.stride(1), dt.stride(0),
-                  dt.stride(1), W.stride(0), B.stride(0), B.stride(1), C.stride(0),
-                  C.stride(1), y.stride(0), y.stride(1), int(chunk), ws.data_ptr(), ws.numel(),
-                  stream)
+                  ptr(h_last), Bsz, L, Dc, N, rank, *sx, dt.stride(0), dt.stride(1), W.stride(0),
+                  *sB, *sC, *sy, int(chunk), ws.data_ptr(), ws.numel(), stream)
     else:
         _lib.call("tssm_selective_scan", code, _disc_code(disc), x.data_ptr(), dt.data_ptr(),
                   int(bool(dt_is_tau)), A_log.data_ptr(), B.data_ptr(), C.data_ptr(), ptr(D),
-                  ptr(h0), y.data_ptr(), ptr(h_last), Bsz, L, Dc, N, x.stride(0), x.stride(1),
-                  *sdt, B.stride(0), B.stride(1), C.stride(0), C.stride(1), y.stride(0),
-                  y.stride(1), int(chunk), ws.data_ptr(), ws.numel(), stream)
+                  ptr(h0), y.data_ptr(), ptr(h_last), Bsz, L, Dc, N, *sx, *sdt, *sB, *sC, *sy,
+                  int(chunk), ws.data_ptr(), ws.numel(), stream)
     return (y, h_last) if return_state else y
 
 

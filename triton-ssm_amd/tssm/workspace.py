@@ -47,6 +47,9 @@ _lock = threading.Lock()
 _cache: dict[tuple[int, int, str], torch.Tensor] = {}
 # pinned host int per lookback workspace (same key), set by a failing kernel
 _host_flags: dict[tuple[int, int, str], torch.Tensor] = {}
+# the same ints as ctypes objects over the tensors' memory: get() polls one on
+# every launch, and reading a tensor element costs a microsecond
+_flag_ints: dict[tuple[int, int, str], ctypes.c_int] = {}
 
 _EXPIRED = ("a bounded look-back wait expired (a predecessor tile never published its "
             "carry); outputs of fused scans since the last check are invalid: ")
@@ -58,9 +61,9 @@ def _dev_index(device: torch.device) -> int:
 
 def _raise_if_flagged(key) -> None:
     """Host-side poll of a workspace's attached flag (no synchronisation)."""
-    flag = _host_flags.get(key)
-    if flag is not None and int(flag[0]) != 0:
-        flag[0] = 0
+    flag = _flag_ints.get(key)
+    if flag is not None and flag.value != 0:
+        flag.value = 0
         raise _lib.TssmError(_EXPIRED + f"device {key[0]} stream {key[1]:#x} (reported by the "
                              "workspace's host flag; the device word stays set for check())")
 
@@ -81,6 +84,7 @@ def get(device: torch.device, stream: int, nbytes: int, kind: str = LOOKBACK) ->
                 if flag is None:
                     flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
                     _host_flags[key] = flag
+                    _flag_ints[key] = ctypes.c_int.from_address(flag.data_ptr())
                 # the header's flag address is written by a synchronous copy,
                 # after the zero fill above
                 _lib.call("tssm_workspace_attach_host_flag", buf.data_ptr(), flag.data_ptr())
@@ -143,4 +147,5 @@ def check(device: torch.device | int | None = None, clear: bool = True) -> None:
 def clear() -> None:
     with _lock:
         _cache.clear()
+        _flag_ints.clear()
         _host_flags.clear()
