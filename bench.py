@@ -10,7 +10,7 @@ x/B/C/y, fp32 dt and state, ZOH discretization fused into the load stage.
   interp_mamba1  interpolation + Mamba-1 scan B=16 T=2048 F=256 N=16 fp32
   ssd_long       SSD scan B=1 L=262144 H=8 P=64 N=16 bf16, chunk 256
   ssd_config1    SSD scan on the headline shapes B=8 L=4096 H=16 P=N=64 bf16
-  ssd_n64_long   SSD scan B=1 L=65536 H=8 P=N=64 bf16 (time-segmented one-pass kernel)
+  ssd_n64_long   SSD scan B=1 L=65536 H=8 P=N=64 bf16 (time-segmented walk)
   ssd_stream     streaming SSD step, 4096 streams H=32 P=64 N=128 fp32 state
   dtproj         Mamba-1 scan B=16 L=2048 D=256 N=16 fp32 with dt = clamp(softplus(
                  dt_raw W + bias)) formed inside the scan's passes (rank 16)
@@ -169,7 +169,7 @@ def wl_ssd_config1(args, dev):
     n = B * L * H * P
     nbytes = 2 * (2 * n + 2 * B * L * H * N) + 4 * B * L * H + 4 * H
     return dict(step=step, cpu=cpu, elements=n, bytes=nbytes,
-                kernel="ssd_seq_kernel", traffic="ssd_seq_traffic.json", dtype="bf16",
+                kernel="ssd_walk16_out_kernel", traffic="ssd_walk16_traffic.json", dtype="bf16",
                 metric="SSD scan elements/sec on the headline shapes, B=8 L=4096 H=16 P=N=64 bf16",
                 unit="elements/s",
                 config={"workload": "SSD scan (decay per head, P x N state) on the DIAG headline "
@@ -548,8 +548,8 @@ def wl_ssd_long(args, dev):
 
 def wl_ssd_n64_long(args, dev):
     """bf16 N = 64 with one row per head and a long sequence (B=1 L=65536 H=8
-    P=N=64): 16 (row, channel block) units, so the one-pass kernel runs 16
-    time segments after the segment end-state and prefix passes."""
+    P=N=64): 16 (row, channel block) units, so the output pass runs 16 time
+    segments after the end-state pass."""
     import torch
     from tssm import ssd_scan_forward, workloads
     w = workloads.ssd_long(L=65536, N=64)
@@ -580,14 +580,14 @@ def wl_ssd_n64_long(args, dev):
     n = B * L * H * P
     nbytes = 2 * (2 * n + 2 * B * L * H * N) + 4 * B * L * H + 4 * H
     return dict(step=step, cpu=cpu, elements=n, bytes=nbytes,
-                kernel="ssd_seg_state_kernel + ssd_seg_prefix_kernel + ssd_seq_kernel",
+                kernel="ssd_walk16_state_kernel + ssd_walk16_out_kernel",
                 traffic="ssd_n64_long_traffic.json",
                 dtype="bf16",
                 metric="SSD long-sequence scan elements/sec, B=1 L=65536 H=8 P=N=64 bf16",
                 unit="elements/s",
                 config={"workload": "SSD scan (decay per head, P x N state), B=1 L=65536 H=8 "
                                     f"P=N=64, chunk {args.ssd_chunk}, bf16 I/O, fp32 state, "
-                                    f"{args.disc.upper()}, time-segmented one-pass kernel",
+                                    f"{args.disc.upper()}, time-segmented walk",
                         "B": B, "L": L, "H": H, "P": P, "N": N, "chunk": args.ssd_chunk})
 
 

@@ -1,6 +1,6 @@
 // Shapes and matrix-core helpers shared by the SSD translation units
 // (ssd.hip: generic passes, N = 16 tile passes, one-launch kernel, streaming
-// step; ssd_n64.hip: the bf16 N = 64 one-pass kernel and its time segments).
+// step; ssd_walk.hip, ssd_walk_bf16.hip: every other form).
 #pragma once
 
 #include "common.h"
@@ -78,18 +78,13 @@ __device__ inline void mfma_step_scalars(const SsdArgs& a, uint32_t h, int64_t t
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-// bf16 N = 64 on the matrix cores (ssd_n64.hip)
-constexpr int kSqQ = 128;  // steps per block
-constexpr int kSqN = 64;   // state size
-constexpr int kSqP = 16;   // channels per product tile (a workgroup takes 1 or 2)
-
-// The bf16 N = 64 one-pass path (ssd_n64.hip) for `rows` rows of P channels:
-// time segments when the rows leave workgroups idle, then the one-pass kernel.
-int launch_ssd_seq_any(int disc, bool has_d, int64_t rows, int64_t P, hipStream_t s,
-                       const SsdArgs& a);
-
 // Every other operand form, with fp32 matrix products (ssd_walk.hip); the
 // workspace is a.chunkX .. a.chunkA + rows x nchunks.
+void launch_ssd_walk_prefix(uint32_t nseg, int64_t PN, hipStream_t s, const SsdArgs& a);
 int launch_ssd_walk(int dtype, int disc, int N, hipStream_t s, const SsdArgs& a);
+
+// bf16 with N = 64 or 32 and 16-byte rows, P a multiple of 8, row strides
+// below 2^25 (ssd_walk_bf16.hip); the same workspace.
+int launch_ssd_walk_bf16(int disc, int N, hipStream_t s, const SsdArgs& a);
 
 }  // namespace tssm

@@ -1,6 +1,6 @@
 // SSD selective scan with fp32 matrix products, for every operand form the
-// bf16 kernels of ssd.hip and ssd_n64.hip do not take (fp32 and fp16, bf16
-// at other head dims and state sizes, any alignment).
+// bf16 kernels of ssd.hip and ssd_walk_bf16.hip do not take (fp32 and fp16,
+// bf16 at other head dims and state sizes, any alignment).
 //
 // One wave owns (row, 16 PB channels, time segment) and walks its segment in
 // 16-step blocks with its slice of the state in registers.  With cum_t the
@@ -15,9 +15,9 @@
 // is the next product's operand where that product runs over k = 4 j + r.  G
 // feeds the x product and H^T feeds the C product that way, with no data moved
 // between lanes.  x, B and C are staged through LDS (a wave's own region, one
-// block; the next one's loads are in flight meanwhile): loads cover whole rows in 16-byte pieces, and the reads take B both
-// by step (G: lane 16 j + c row c) and by state column (the update: column
-// 16 i + c).  Operands loaded straight from memory in their lane order, with
+// block; the next one's loads are in flight meanwhile): loads cover whole rows
+// in 16-byte pieces, and the reads take B both by step (G: lane 16 j + c row c)
+// and by state column (the update: column 16 i + c).  Operands loaded straight from memory in their lane order, with
 // neighbouring lanes on different rows, cost the first-level cache ~1000
 // accesses a block instead of ~160, and twice the waves then ran slower (75
 // against 66 us); two blocks in LDS leave room for one wave a SIMD (105
@@ -41,25 +41,12 @@
 // has underflowed to exactly zero; ssd_walk_prefix_kernel turns them into
 // entry states; ssd_walk_out_kernel writes the outputs.  One segment takes the last
 // kernel alone.
-#include "ssd_dev.h"
-
-#include <type_traits>
+#include "ssd_walk_dev.h"
 
 namespace tssm {
 namespace {
 
-constexpr int kWalkQ = 16;           // steps per block
-constexpr double kWalkFloor = -4096; // log2 decay of one step, clamped: 2^-4096 is 0 either way
-
-// Lane i of each 16-lane row gets lane i - n (row_shr), 0.0 before the row.
-template <int CTRL>
-__device__ inline double dpp_shr_f64(double v) {
-  const u32x2 w = __builtin_bit_cast(u32x2, v);
-  u32x2 r;
-  r[0] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w[0], CTRL, 0xf, 0xf, true);
-  r[1] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w[1], CTRL, 0xf, 0xf, true);
-  return __builtin_bit_cast(double, r);
-}
+constexpr int kWalkQ = 16;  // steps per block
 
 // The step scalars of one block.  Lane 16 j + c: cum, coef of step c; cs, cf
 // those of steps 4 j + r; cum_e the sum over the block (uniform).
@@ -95,179 +82,6 @@ __device__ inline WalkScalars walk_scalars(float d, float a2, double a2d, bool z
   return o;
 }
 
-// What a wave works on.  Waves of one (batch, segment) share the 128-byte
-// lines of dt, so with enough (batch, segment) groups their workgroups are
-// numbered onto one XCD (blockIdx mod 8).
-struct WalkUnit {
-  uint32_t b, h, row, seg;
-  int p0;
-  bool on;
-};
-__device__ inline WalkUnit walk_unit(const SsdArgs& a, uint32_t npg, uint32_t nseg, int pw,
-                                     bool by_xcd) {
-  const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t per = a.H * npg;  // waves per (batch, segment)
-  const uint32_t groups = a.rows / a.H * nseg;
-  uint32_t g, u;
-  if (by_xcd) {
-    const uint32_t wgs = (per + 3) / 4, idx = blockIdx.x >> 3;
-    g = (idx / wgs) * 8 + (blockIdx.x & 7);
-    u = (idx % wgs) * 4 + wv;
-  } else {
-    const uint32_t w = blockIdx.x * 4 + wv;
-    g = w / per;
-    u = w - g * per;
-  }
-  WalkUnit o;
-  o.on = g < groups && u < per;
-  o.b = g / nseg;
-  o.seg = g - o.b * nseg;
-  o.h = u / npg;
-  o.p0 = (int)(u - o.h * npg) * pw;
-  o.row = o.b * a.H + o.h;
-  return o;
-}
-
-typedef f32x4 mfma_acc;
-__device__ inline mfma_acc mfma4(float a, float b, mfma_acc c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// Orders a wave's LDS writes before its other lanes' reads (the LDS itself
-// runs a wave's accesses in order: no instruction).
-__device__ inline void wave_lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// One staged operand: 16 rows (steps) of 16 WB columns.  In LDS a row takes
-// 16 bytes more than its columns, so that the rows c of a vector read and the
-// rows 4 j + r of an element read fall on different banks.
-template <typename T, int WB, bool VEC>
-struct WalkTile {
-  static constexpr int E = (int)sizeof(T), W = 16 * WB, kStride = W * E + 16;
-  static constexpr int kBytes = kWalkQ * kStride;
-  static constexpr int VE = VEC ? 16 / E : 1;  // elements of one access
-  static constexpr int NP = W / VE;            // accesses of a row
-  static constexpr int K = (kWalkQ * NP + 63) / 64;
-  typedef std::conditional_t<VEC, uint32_t, uint64_t> off_t;
-  typedef std::conditional_t<VEC, u32x4, uint32_t> raw_t;
-  struct Regs {
-    raw_t v[K];
-  };
-  off_t off[K];
-  int lim;  // columns that exist (the others are zero)
-  static __device__ inline int row_of(int lane, int k) { return (lane + 64 * k) / NP % kWalkQ; }
-  static __device__ inline int col_of(int lane, int k) { return (lane + 64 * k) % NP * VE; }
-  // Byte offsets from the block's first row; rows past `last` re-read it.
-  __device__ inline void rows(int lane, int64_t stride, int last) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const int r = row_of(lane, k), c = col_of(lane, k);
-      off[k] = (off_t)(r < last ? r : last) * (off_t)stride + (off_t)((c < lim ? c : 0) * E);
-    }
-  }
-  __device__ inline void load(Regs& g, const char* base) const {
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      if constexpr (VEC) g.v[k] = *reinterpret_cast<const u32x4*>(base + off[k]);
-      else if constexpr (E == 4) g.v[k] = *reinterpret_cast<const uint32_t*>(base + off[k]);
-      else g.v[k] = *reinterpret_cast<const uint16_t*>(base + off[k]);
-    }
-  }
-  // Columns past lim and rows past `n` are stored as zero.
-  __device__ inline void store(Regs& g, char* lds, int lane, bool edge, int n) const {
-    if (edge) {
-#pragma unroll
-      for (int k = 0; k < K; ++k)
-        g.v[k] &= row_of(lane, k) < n && col_of(lane, k) < lim ? ~0u : 0u;
-    }
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      char* p = lds + row_of(lane, k) * kStride + col_of(lane, k) * E;
-      if constexpr (VEC) *reinterpret_cast<u32x4*>(p) = g.v[k];
-      else if constexpr (E == 4) *reinterpret_cast<uint32_t*>(p) = g.v[k];
-      else *reinterpret_cast<uint16_t*>(p) = (uint16_t)g.v[k];
-    }
-  }
-  static __device__ inline float get(const char* lds, int row, int col) {
-    return ldf(reinterpret_cast<const T*>(lds + row * kStride + col * E));
-  }
-  static __device__ inline void get4(const char* lds, int row, int col, float* o) {
-    ld_lanes<T, 4>(reinterpret_cast<const T*>(lds + row * kStride + col * E), o);
-  }
-};
-
-// The operands of a wave: a block in LDS, the next one's loads in flight.
-template <typename T, int PB, int NB, bool VEC, bool OUT>
-struct WalkIn {
-  typedef WalkTile<T, PB, VEC> TX;
-  typedef WalkTile<T, NB, VEC> TN;
-  static constexpr int kX = 0, kB = TX::kBytes, kC = kB + TN::kBytes;
-  static constexpr int kBytes = OUT ? kC + TN::kBytes : kC;
-  // the registers of one block's loads
-  struct Regs {
-    typename TX::Regs x;
-    typename TN::Regs B, C;
-    float dt;
-  };
-  TX x;
-  TN B, C;
-  const char *px, *pB, *pC, *pd;  // (batch, head) bases
-  int64_t L, sx, sB, sC, sdt;     // row strides in bytes
-  typename TX::off_t od;
-  bool edge;                      // some columns do not exist
-  int lane;
-  __device__ inline void rows(int last) {
-    const int c = lane & 15;
-    x.rows(lane, sx, last);
-    B.rows(lane, sB, last);
-    if constexpr (OUT) C.rows(lane, sC, last);
-    od = (typename TX::off_t)(c < last ? c : last) * (typename TX::off_t)sdt;
-  }
-  __device__ inline void init(const SsdArgs& a, const WalkUnit& u, int N, int ln) {
-    lane = ln;
-    px = reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.x) + u.b * a.sx_b +
-                                       u.h * a.sx_h + u.p0);
-    pB = reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.B) + u.b * a.sB_b +
-                                       u.h * a.sB_h);
-    pC = reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.C) + u.b * a.sC_b +
-                                       u.h * a.sC_h);
-    pd = reinterpret_cast<const char*>(a.dt + u.b * a.sdt_b + u.h * a.sdt_h);
-    L = a.L;
-    sx = a.sx_l * (int64_t)sizeof(T);
-    sB = a.sB_l * (int64_t)sizeof(T);
-    sC = a.sC_l * (int64_t)sizeof(T);
-    sdt = a.sdt_l * 4;
-    x.lim = (int)a.P - u.p0 < TX::W ? (int)a.P - u.p0 : TX::W;
-    B.lim = C.lim = N;
-    edge = x.lim < TX::W || N < TN::W;
-    rows(kWalkQ - 1);
-  }
-  __device__ inline void load(Regs& g, int64_t t0) {
-    const int64_t tb = t0 < L ? t0 : L - 1;
-    if (tb + kWalkQ > L) rows((int)(L - 1 - tb));
-    g.dt = *reinterpret_cast<const float*>(pd + tb * sdt + od);
-    x.load(g.x, px + tb * sx);
-    B.load(g.B, pB + tb * sB);
-    if constexpr (OUT) C.load(g.C, pC + tb * sC);
-  }
-  // The loaded block, whose first step is t0, into LDS; returns the dt of step
-  // t0 + lane % 16 (0 past the end).
-  __device__ inline float stage(Regs& g, char* lds, int64_t t0) const {
-    const int64_t left = L - t0;
-    const int n = left < kWalkQ ? (left > 0 ? (int)left : 0) : kWalkQ;
-    const bool e = edge || n < kWalkQ;
-    wave_lds_order();  // after the reads of the block before
-    x.store(g.x, lds + kX, lane, e, n);
-    B.store(g.B, lds + kB, lane, e, n);
-    if constexpr (OUT) C.store(g.C, lds + kC, lane, e, n);
-    wave_lds_order();
-    return (lane & 15) < n ? g.dt : 0.0f;
-  }
-};
-
 // H^T += sum_s w_s B_s x_s^T over one block, w[r] the weight of step 4 j + r,
 // xv its channels 16 q + c.
 template <typename In, int PB, int NB>
@@ -284,30 +98,12 @@ __device__ inline void walk_update(mfma_acc (&H)[NB][PB], const char* lds, const
   }
 }
 
-// H^T[i][q] reg r  <->  S[p][n], n = 16 i + 4 j + r, p = p0 + 16 q + c.
-template <int PB, int NB>
-__device__ inline void walk_put(float* S, const mfma_acc (&H)[NB][PB], int p0, int P, int N, int c,
-                                int j) {
-#pragma unroll
-  for (int q = 0; q < PB; ++q) {
-    const int p = p0 + 16 * q + c;
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int n0 = 16 * i + 4 * j;
-      if (p < P && n0 < N) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) S[(int64_t)p * N + n0 + r] = H[i][q][r];
-      }
-    }
-  }
-}
-
 // Pass 1: end state from zero and decay of segment seg < nseg - 1.
 template <typename T, int PB, int NB, bool VEC>
 __global__ __launch_bounds__(256) void ssd_walk_state_kernel(SsdArgs a, int N, uint32_t npg,
                                                              uint32_t nsub, uint32_t segb, int zoh,
                                                              int by_xcd) {
-  typedef WalkIn<T, PB, NB, VEC, false> In;
+  typedef WalkIn<T, PB, NB, VEC, false, kWalkQ> In;
   __shared__ __align__(16) char s_in[4][In::kBytes];
   const int lane = threadIdx.x & 63, c = lane & 15, j = lane >> 4;
   const WalkUnit u = walk_unit(a, npg, nsub, 16 * PB, by_xcd != 0);
@@ -354,7 +150,7 @@ __global__ __launch_bounds__(256) void ssd_walk_state_kernel(SsdArgs a, int N, u
 template <typename T, int PB, int NB, bool VEC, bool HAS_D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void ssd_walk_out_kernel(
     SsdArgs a, int N, uint32_t npg, uint32_t nseg, uint32_t segb, int zoh, int by_xcd) {
-  typedef WalkIn<T, PB, NB, VEC, true> In;
+  typedef WalkIn<T, PB, NB, VEC, true, kWalkQ> In;
   __shared__ __align__(16) char s_in[4][In::kBytes];
   const int lane = threadIdx.x & 63, c = lane & 15, j = lane >> 4;
   const int P = (int)a.P;
@@ -374,33 +170,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   const float* hin = nseg > 1 ? a.chunkX + ((int64_t)u.row * nseg + u.seg) * PN
                               : (a.h0 ? a.h0 + (int64_t)u.row * PN : nullptr);
   mfma_acc H[NB][PB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i)
-#pragma unroll
-    for (int q = 0; q < PB; ++q) H[i][q] = mfma_acc{0.0f, 0.0f, 0.0f, 0.0f};
-  if (hin) {
-    // loads first (lanes past P or N re-read the slice's start), zeroes by
-    // mask: the compiler turns a select on a loaded value into a branch around
-    // the load, which then waits for it alone
-#pragma unroll
-    for (int q = 0; q < PB; ++q)
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        const int p = u.p0 + 16 * q + c, n0 = 16 * i + 4 * j;
-        const float* hp = hin + (p < P ? p : 0) * N + (n0 < N ? n0 : 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) H[i][q][r] = hp[r];
-      }
-#pragma unroll
-    for (int q = 0; q < PB; ++q)
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        const uint32_t m = u.p0 + 16 * q + c < P && 16 * i + 4 * j < N ? ~0u : 0u;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          H[i][q][r] = __uint_as_float(__float_as_uint(H[i][q][r]) & m);
-      }
-  }
+  walk_get<PB, NB>(H, hin, u.p0, P, N, c, j);
   // outputs: lane (c = step, j) holds channels po + 16 q + r
   const int po = u.p0 + 4 * j;
   T* yp = reinterpret_cast<T*>(a.y) + u.b * a.sy_b + u.h * a.sy_h + po;
@@ -549,6 +319,15 @@ __global__ __launch_bounds__(256) void ssd_walk_prefix_kernel(SsdArgs a, uint32_
   }
 }
 
+}  // namespace
+
+void launch_ssd_walk_prefix(uint32_t nseg, int64_t PN, hipStream_t s, const SsdArgs& a) {
+  hipLaunchKernelGGL(ssd_walk_prefix_kernel, dim3((unsigned)cdiv64(a.rows * PN, 256)), dim3(256), 0,
+                     s, a, nseg, PN);
+}
+
+namespace {
+
 struct WalkPlan {
   int pb;
   uint32_t npg, nseg, segb;
@@ -594,21 +373,13 @@ int launch_walk(const WalkPlan& pl, int disc, int N, hipStream_t s, SsdArgs a) {
   a.chunkA = a.chunkX + (int64_t)a.rows * pl.nseg * a.P * N;
   const int64_t per = (int64_t)a.H * pl.npg, nbatch = a.rows / a.H;
   const int zoh = disc == TSSM_DISC_ZOH;
-  auto grid = [&](int64_t nseg, int* by_xcd) {
-    const int64_t groups = nbatch * nseg;
-    // an uneven split over the XCDs costs more than sharing dt's lines gains
-    *by_xcd = groups % 8 == 0 || groups >= 64;
-    return *by_xcd ? dim3((unsigned)(8 * cdiv64(groups, 8) * cdiv64(per, 4)))
-                   : dim3((unsigned)cdiv64(groups * per, 4));
-  };
+  auto grid = [&](int64_t nseg, int* by_xcd) { return walk_grid(nbatch * nseg, per, by_xcd); };
   int bx = 0;
   if (pl.nseg > 1) {
     const dim3 g1 = grid(pl.nseg - 1, &bx);
     hipLaunchKernelGGL((ssd_walk_state_kernel<T, PB, NB, VEC>), g1, dim3(256), 0, s, a, N, pl.npg,
                        pl.nseg - 1, pl.segb, zoh, bx);
-    const int64_t PN = (int64_t)a.P * N;
-    hipLaunchKernelGGL(ssd_walk_prefix_kernel, dim3((unsigned)cdiv64(a.rows * PN, 256)), dim3(256),
-                       0, s, a, pl.nseg, PN);
+    launch_ssd_walk_prefix(pl.nseg, (int64_t)a.P * N, s, a);
   }
   const dim3 g3 = grid(pl.nseg, &bx);
   if (a.D)
