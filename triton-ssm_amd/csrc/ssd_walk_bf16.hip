@@ -29,13 +29,12 @@
 //
 // Bound by the chain of dependent phases with one workgroup (two waves a SIMD) on a
 // CU, not by HBM: B=8 L=4096 H=16 P=N=64 takes 86.9 us with 271 MB moved (the one-pass
-// kernel it replaced: 101.1), about 53 at a copy's rate; a
-// super-block of 8 x 32 steps costs a wave 10,200 cycles, no phase over a fifth.
+// kernel it replaced: 101.1), about 53 at a copy's rate.  A super-block of 8 x 32
+// steps cost a wave 10,200 cycles while the decays were summed in fp64 (90 us), no
+// phase over a fifth of them.
 // B=1 L=65536 H=8: 119.8 us a call (before 139 - 144); N = 32, B=8 L=4096 H=16 P=64,
 // 55 us (the vector passes took 321).  16 channels a wave measured 115 - 129 us on
-// the first shape, 12 waves a workgroup 118 (spills).  Where segments are few and
-// decays slow the state pass costs more than it gives: B=1 L=20000 H=1, step sizes
-// x 0.003, 33.1 us against 29.2; with ordinary ones 23.3 against 27.8.
+// the first shape, 12 waves a workgroup 118 (spills).
 #include "ssd_walk_dev.h"
 
 namespace tssm {
@@ -506,8 +505,11 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
 // memory).  Pass 1 takes a segment in m sub-segments of at least
 // kW16MinSub blocks, up to two of its waves a SIMD: with slow decays it walks
 // all of them (B=1 L=65536 H=8 P=N=64, slow decays: 190 us with m = 1, 132 with
-// m = 8).
-constexpr int64_t kW16MinSuper = 2, kW16StateWaves = 2048, kW16MinSub = 8;
+// m = 8), and no more of them than the output pass folds itself (B=1 L=100000
+// H=1: 53 us with 389 and the prefix pass, 30 with 98; slow decays 59 and 53).
+// Segments of one super-block beat two where units are few: B=1 L=20000 H=1
+// 23.5 -> 19.8 us, slow decays 33.2 -> 29.6; L=700 pays, 15.8 -> 16.6.
+constexpr int64_t kW16MinSuper = 1, kW16StateWaves = 2048, kW16MinSub = 8;
 template <int PB, int NB>
 int launch_walk16(int disc, hipStream_t s, SsdArgs a) {
   constexpr int N = 16 * NB;
@@ -526,7 +528,8 @@ int launch_walk16(int disc, hipStream_t s, SsdArgs a) {
   nseg = cdiv64(nblk, segb);
   int64_t m = 1;
   while (segb % (2 * m) == 0 && segb / (2 * m) >= kW16MinSub &&
-         units * (nseg - 1) * 2 * m <= kW16StateWaves && (nseg - 1) * 2 * m + 1 <= cap)
+         units * (nseg - 1) * 2 * m <= kW16StateWaves && (nseg - 1) * 2 * m + 1 <= cap &&
+         (nseg - 1) * 2 * m + 1 <= kW16Fold)
     m *= 2;
   const int64_t nslot = (nseg - 1) * m + 1;
   a.chunkA = a.chunkX + (int64_t)a.rows * nslot * PN;
