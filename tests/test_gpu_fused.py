@@ -636,6 +636,39 @@ def test_selective_scan(dev, dtype, N, Dc, dt_per_channel):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,L,Dc,N,disc,dt_form,extras", [
+    (64, 64, 300, 16, "zoh", "channel", True), (64, 65, 300, 16, "euler", "shared", False),
+    (16, 520, 70, 16, "zoh", "tau", True), (32, 127, 257, 8, "zoh", "shared", True),
+    (64, 300, 40, 8, "euler", "channel", False), (9, 300, 512, 16, "zoh", "channel", True),
+    (40, 96, 257, 8, "euler", "tau", True)])
+def test_selective_scan_walk(dev, dtype, B, L, Dc, N, disc, dt_form, extras):
+    """The one-sweep Mamba-1 scan at the edges of its 64-step tiles and 16-channel
+    groups, each form of dt, rows inside wider tensors.  bf16: the output's rounding
+    (2^-9 of a value) is the only one, well inside 4e-3 of the largest."""
+    from tssm import selective_scan_forward
+    d = _mamba1_inputs(dev, B, L, Dc, N, dtype, seed=L + Dc, dt_per_channel=dt_form == "channel")
+    tau = dt_form == "tau"
+    dt = d["dt"].cumsum(1) if tau else d["dt"]
+    wide = torch.zeros(B, L, Dc + 3, device=dev, dtype=dtype)
+    wide[..., 1:Dc + 1] = d["x"]
+    x = wide[..., 1:Dc + 1]
+    h0 = torch.randn(B, Dc, N, device=dev) if extras else None
+    D = d["D"] if extras else None
+    y, h = selective_scan_forward(x, dt, d["A_log"], d["B"], d["C"], D, h0=h0, disc=disc,
+                                  dt_is_tau=tau, return_state=True)
+    steps = np.diff(np64(dt), axis=1, prepend=0.0) if tau else np64(dt)
+    y_ref, h_ref = O.selective_scan(np64(x), steps, d["A_log"], d["B"], d["C"], D,
+                                    h0=None if h0 is None else np64(h0), disc=disc)
+    # differences of timestamps are taken in fp32: at most 2^-24 of the last one
+    # against a step, weighted by the largest |a|
+    slack = 0.0
+    if tau:
+        slack = 2.0 ** -23 * float(np64(dt).max()) * float(np.exp(np64(d["A_log"])).max())
+    assert_close(y, y_ref, (1e-5 if dtype == torch.float32 else 4e-3) + slack, "walk y")
+    assert_close(h, h_ref, 1e-5 + slack, "walk h_last")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("N,Dc,rank,L", [(16, 40, 16, 700), (8, 24, 1, 333), (64, 6, 33, 520),
                                          (16, 256, 64, 300), (32, 9, 4, 129), (128, 3, 7, 200)])
 def test_selective_scan_dtproj(dev, dtype, N, Dc, rank, L):

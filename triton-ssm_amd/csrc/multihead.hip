@@ -1376,6 +1376,10 @@ int selective_scan_launch(int dtype, int disc, const void* x, const float* dt, i
       SelPtrs p;
       p.x = x; p.dt = dt; p.A_log = A_log; p.B = B; p.C = C; p.D = D; p.h0 = h0; p.y = y;
       p.h_last = h_last;
+      if (!proj.W && sel_walk_ok(nbatch, L, Dc, N, dt_shared, sx_l, sdt_l, sdt_d, sB_l, sC_l))
+        return sel_walk_launch(dtype, disc, dt_shared, dt_is_tau != 0, p, nbatch, L, Dc, N, sx_b,
+                               sx_l, sdt_b, sdt_l, sdt_d, sB_b, sB_l, sC_b, sC_l, sy_b, sy_l,
+                               as_stream(stream));
       p.W = proj.W; p.bias = proj.bias; p.sw_r = proj.sw_r; p.rank = proj.rank;
       p.dt_min = proj.dt_min; p.dt_max = proj.dt_max;
       const int64_t off = sel_chunked_offset(sel_lookback_bytes(nbatch, L, Dc, N, chunk));

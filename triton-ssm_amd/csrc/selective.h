@@ -74,6 +74,17 @@ int sel_chunked_launch(int dtype, int disc, bool dt_shared, bool tau, const SelP
                        int64_t sB_l, int64_t sC_b, int64_t sC_l, int64_t sy_b, int64_t sy_l,
                        hipStream_t s);
 
+// The one-sweep scan (sel_walk.hip): one lane per (batch, channel, state), N = 8 or
+// 16, fp32 or bf16, dt given.  sel_walk_ok says whether it is the faster one for a
+// problem that would take the passes.
+bool sel_walk_ok(int64_t nbatch, int64_t L, int64_t Dc, int64_t N, bool dt_shared,
+                 int64_t sx_l, int64_t sdt_l, int64_t sdt_d, int64_t sB_l, int64_t sC_l);
+// Uses x, dt, A_log, B, C, D, h0, y and h_last of `p`; no workspace.
+int sel_walk_launch(int dtype, int disc, bool dt_shared, bool tau, const SelPtrs& p,
+                    int64_t nbatch, int64_t L, int64_t Dc, int64_t N, int64_t sx_b, int64_t sx_l,
+                    int64_t sdt_b, int64_t sdt_l, int64_t sdt_d, int64_t sB_b, int64_t sB_l,
+                    int64_t sC_b, int64_t sC_l, int64_t sy_b, int64_t sy_l, hipStream_t s);
+
 // Whether the interpolation can be formed inside pass 1 (sel_interp_launch):
 // fp32/bf16 I/O, N 8 or 16, fp32 masks in 16-byte rows, FTILE a power of two
 // in [16, 256], 1 <= K <= 64, F a multiple of 4, a problem the three passes
