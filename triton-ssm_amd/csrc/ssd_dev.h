@@ -83,8 +83,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 void launch_ssd_walk_prefix(uint32_t nseg, int64_t PN, hipStream_t s, const SsdArgs& a);
 int launch_ssd_walk(int dtype, int disc, int N, hipStream_t s, const SsdArgs& a);
 
-// bf16 with N = 64 or 32 and 16-byte rows, P a multiple of 8, row strides
-// below 2^25 (ssd_walk_bf16.hip); the same workspace.
-int launch_ssd_walk_bf16(int disc, int N, hipStream_t s, const SsdArgs& a);
+// bf16 with N = 64, P a multiple of 16, 16-byte rows and row strides below 2^25
+// (ssd_walk_bf16.hip); the same workspace.
+int launch_ssd_walk_bf16(int disc, hipStream_t s, const SsdArgs& a);
 
 }  // namespace tssm

@@ -1,5 +1,5 @@
-// SSD selective scan, bf16 with N = 64 (and 32), on the bf16 matrix cores: the
-// walk of ssd_walk.hip with 32-step blocks and K = 32 products.
+// SSD selective scan, bf16 with N = 64 and P a multiple of 16, on the bf16 matrix
+// cores: the walk of ssd_walk.hip with 32-step blocks and K = 32 products.
 //
 // A unit is (row, 32 channels, time segment).  In the state pass one wave owns a
 // unit; in the output pass a workgroup of 8 waves takes 8 blocks of it at a time:
@@ -32,15 +32,21 @@
 // kernel it replaced: 101.1), about 53 at a copy's rate.  A super-block of 8 x 32
 // steps cost a wave 10,200 cycles while the decays were summed in fp64 (90 us), no
 // phase over a fifth of them.
-// B=1 L=65536 H=8: 119.8 us a call (before 139 - 144); N = 32, B=8 L=4096 H=16 P=64,
-// 55 us (the vector passes took 321).  16 channels a wave measured 115 - 129 us on
-// the first shape, 12 waves a workgroup 118 (spills).
+// B=1 L=65536 H=8: 119.8 us a call (before 139 - 144).  16 channels a wave measured
+// 115 - 129 us on the first shape, 12 waves a workgroup 118 (spills).
+//
+// The hi/lo operands keep 16 bits, which y's rounding hides and the fp32 final
+// state does not: 2.2e-6 of float64 on it, where fp32 products give 1e-7.  So bf16
+// at other head dims and state sizes, whose state is formed in fp32 throughout, is
+// not taken here, though N = 32 would run in 55 us instead of 104 (B=8 L=4096 H=16
+// P=64).
 #include "ssd_walk_dev.h"
 
 namespace tssm {
 namespace {
 
 constexpr int kW16Q = 32;  // steps per block
+constexpr int NB = 4;      // column tiles of 16: N = 64
 // Most sub-segments whose end states the output pass folds into entry states
 // itself; more take the prefix pass.  Folding reads eight states where decays
 // forget and 15 rounds of eight at worst, the prefix pass 10-18 us either way.
@@ -103,7 +109,7 @@ __device__ inline W16Steps w16_steps(float d, float a2, bool zoh) {
 
 // H^T += sum_s w_s B_s x_s^T over the block's 32 steps: w the LDS weights,
 // xc the x columns read_cols gave for (half a, channel block q).
-template <typename In, int PB, int NB>
+template <typename In, int PB>
 __device__ inline void w16_update(mfma_acc (&H)[NB][PB], const char* lds, const float* w,
                                   const s16x4_t (&xc)[2][PB], int c, int j) {
   bf16x8_t xh[PB], xl[PB];
@@ -139,7 +145,7 @@ __device__ inline void w16_update(mfma_acc (&H)[NB][PB], const char* lds, const 
 // Pass 1: end state from zero and decay of each of the `nsub` sub-segments (segb
 // blocks) before the last segment, last block first, stopping once the decay
 // has underflowed to exactly zero.
-template <int PB, int NB>
+template <int PB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void
 ssd_walk16_state_kernel(SsdArgs a, uint32_t npg, uint32_t nsub, uint32_t segb, int zoh,
                         int by_xcd) {
@@ -179,7 +185,7 @@ ssd_walk16_state_kernel(SsdArgs a, uint32_t npg, uint32_t nsub, uint32_t segb, i
 #pragma unroll
       for (int q = 0; q < PB; ++q)
         xc[h][q] = read_cols<typename In::TX>(lds + In::kX, h, 16 * q, c, j);
-    w16_update<In, PB, NB>(H, lds, w, xc, c, j);
+    w16_update<In, PB>(H, lds, w, xc, c, j);
     lsum += s.tot0 + s.tot1;
     return exp2_fast(lsum) != 0.0f;  // uniform; at 0 every earlier weight is zero too
   };
@@ -206,7 +212,7 @@ struct __align__(16) W16Weights {
 // run side by side with one read of the inputs.  A wave's region in LDS holds
 // its staged block, then (every operand taken into registers) the state.
 constexpr int kW16Waves = 8;
-template <int PB, int NB, bool HAS_D>
+template <int PB, bool HAS_D>
 __global__ __launch_bounds__(64 * kW16Waves) __attribute__((amdgpu_waves_per_eu(2))) void
 ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uint32_t m, int zoh) {
   typedef WalkIn<bf16_t, PB, NB, true, true, kW16Q> In;
@@ -347,7 +353,7 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int q = 0; q < PB; ++q) H[i][q] = mfma_acc{0.0f, 0.0f, 0.0f, 0.0f};
-    w16_update<In, PB, NB>(H, lds, sc.wu, xc, c, j);
+    w16_update<In, PB>(H, lds, sc.wu, xc, c, j);
     // the next block's loads, a part at a time: eight waves issuing all of
     // theirs at once wait on each other
     const int64_t tn = in.row0(t0 + kSuper);
@@ -498,11 +504,9 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
   }
 }
 
-// Time segments: as many as fill every CU once (at N = 32, whose LDS leaves room
-// for two workgroups, twice where that gives three segments or more: B=5 L=7604
-// H=13 P=64 95 -> 87 us, but B=8 L=4096 H=16 56 -> 66), each of at least kW16MinSuper super-blocks (a
-// segment costs pass 1 over its end, a launch, and its state twice through
-// memory).  Pass 1 takes a segment in m sub-segments of at least
+// Time segments: as many as fill every CU once, each of at least kW16MinSuper
+// super-blocks (a segment costs pass 1 over its end, a launch, and its state twice
+// through memory).  Pass 1 takes a segment in m sub-segments of at least
 // kW16MinSub blocks, up to two of its waves a SIMD: with slow decays it walks
 // all of them (B=1 L=65536 H=8 P=N=64, slow decays: 190 us with m = 1, 132 with
 // m = 8), and no more of them than the output pass folds itself (B=1 L=100000
@@ -510,16 +514,15 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
 // Segments of one super-block beat two where units are few: B=1 L=20000 H=1
 // 23.5 -> 19.8 us, slow decays 33.2 -> 29.6; L=700 pays, 15.8 -> 16.6.
 constexpr int64_t kW16MinSuper = 1, kW16StateWaves = 2048, kW16MinSub = 8;
-template <int PB, int NB>
+template <int PB>
 int launch_walk16(int disc, hipStream_t s, SsdArgs a) {
-  constexpr int N = 16 * NB;
-  const int64_t PN = (int64_t)a.P * N, nblk = cdiv64(a.L, kW16Q), npg = cdiv64(a.P, 16 * PB);
+  const int64_t PN = (int64_t)a.P * (16 * NB), nblk = cdiv64(a.L, kW16Q), npg = cdiv64(a.P, 16 * PB);
   const int64_t units = (int64_t)a.rows * npg;
   // a slot takes one state and one decay of the workspace, which holds two
   // states and a decay per chunk
   const int64_t cap = (int64_t)a.nchunks * (2 * PN + 1) / (PN + 1);
   const int64_t by_len = nblk / (kW16MinSuper * kW16Waves);
-  int64_t nseg = NB == 2 && 512 / units >= 3 ? 512 / units : 256 / units;
+  int64_t nseg = 256 / units;
   nseg = nseg < cap ? nseg : cap;
   nseg = nseg < by_len ? nseg : by_len;
   if (nseg < 1) nseg = 1;
@@ -538,26 +541,24 @@ int launch_walk16(int disc, hipStream_t s, SsdArgs a) {
   if (nseg > 1) {
     int bx = 0;
     const dim3 g1 = walk_grid(nbatch * (nslot - 1), per, &bx);
-    hipLaunchKernelGGL((ssd_walk16_state_kernel<PB, NB>), g1, dim3(256), 0, s, a, (uint32_t)npg,
+    hipLaunchKernelGGL((ssd_walk16_state_kernel<PB>), g1, dim3(256), 0, s, a, (uint32_t)npg,
                        (uint32_t)(nslot - 1), (uint32_t)(segb / m), zoh, bx);
     if (nslot > kW16Fold) launch_ssd_walk_prefix((uint32_t)nslot, PN, s, a);
   }
   const dim3 g3((unsigned)(nbatch * nseg * per));
   if (a.D)
-    hipLaunchKernelGGL((ssd_walk16_out_kernel<PB, NB, true>), g3, dim3(64 * kW16Waves), 0, s, a,
+    hipLaunchKernelGGL((ssd_walk16_out_kernel<PB, true>), g3, dim3(64 * kW16Waves), 0, s, a,
                        (uint32_t)npg, (uint32_t)nseg, (uint32_t)segb, (uint32_t)m, zoh);
   else
-    hipLaunchKernelGGL((ssd_walk16_out_kernel<PB, NB, false>), g3, dim3(64 * kW16Waves), 0, s, a,
+    hipLaunchKernelGGL((ssd_walk16_out_kernel<PB, false>), g3, dim3(64 * kW16Waves), 0, s, a,
                        (uint32_t)npg, (uint32_t)nseg, (uint32_t)segb, (uint32_t)m, zoh);
   return launch_status();
 }
 
 }  // namespace
 
-int launch_ssd_walk_bf16(int disc, int N, hipStream_t s, const SsdArgs& a) {
-  const bool wide = a.P > 16;
-  if (N == 64) return wide ? launch_walk16<2, 4>(disc, s, a) : launch_walk16<1, 4>(disc, s, a);
-  return wide ? launch_walk16<2, 2>(disc, s, a) : launch_walk16<1, 2>(disc, s, a);
+int launch_ssd_walk_bf16(int disc, hipStream_t s, const SsdArgs& a) {
+  return a.P > 16 ? launch_walk16<2>(disc, s, a) : launch_walk16<1>(disc, s, a);
 }
 
 }  // namespace tssm
