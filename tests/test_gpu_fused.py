@@ -115,6 +115,45 @@ def test_ssd_scan_bf16_walk(dev, B, L, H, P, N, chunk, decay, with_d):
     assert_close(hl, h_ref, 1e-3 if N == 64 and P % 16 == 0 else 2e-6, "bf16 walk h_last")
 
 
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("L,s", [(300, 151), (300, 15), (300, 32), (2000, 1111)])
+@pytest.mark.parametrize("P,N", [(64, 64), (16, 64), (24, 64), (32, 32)])
+def test_ssd_scan_bf16_not_finite(dev, P, N, L, s, value):
+    """bf16: an x that is not finite at step s of one channel leaves every earlier
+    output and every other channel as it was, bit for bit, and reaches that
+    channel's outputs and state from step s on (slow decays: no weight is zero);
+    an infinite one makes that state infinite, and an infinite entry of h0 the
+    outputs (N = 64 with P a multiple of 16 carries the state between blocks as
+    hi/lo parts, where they are NaN)."""
+    from tssm import ssd_scan_forward
+    d = _ssd_inputs(dev, 1, L, 2, P, N, torch.bfloat16, seed=L + P, heavy=False)
+    d["dt"] = d["dt"] * 0.003
+    h0 = torch.randn(1, 2, P, N, device=dev)
+    run = lambda x, h: ssd_scan_forward(x, d["dt"], d["A_log"], d["B"], d["C"], h0=h,  # noqa: E731
+                                        return_state=True)
+    y, hl = run(d["x"], h0)
+    x = d["x"].clone()
+    x[:, s, 1, 5] = value
+    bad, hb = run(x, h0)
+    torch.testing.assert_close(bad[:, :s], y[:, :s], rtol=0, atol=0)
+    rest = [p for p in range(P) if p != 5]
+    torch.testing.assert_close(bad[:, :, 1, rest], y[:, :, 1, rest], rtol=0, atol=0)
+    torch.testing.assert_close(bad[:, :, 0], y[:, :, 0], rtol=0, atol=0)
+    assert not bool(torch.isfinite(bad[:, s:, 1, 5]).any())
+    assert not bool(torch.isfinite(hb[:, 1, 5]).any())
+    if value == float("inf"):
+        assert torch.equal(hb[0, 1, 5], value * torch.sign(d["B"][0, s, 1].float()))
+        h1 = h0.clone()
+        h1[0, 1, 5, 3] = value
+        bad, hb = run(d["x"], h1)
+        if N == 64 and P % 16 == 0:
+            assert not bool(torch.isfinite(bad[0, :, 1, 5]).any())
+        else:
+            assert torch.equal(bad[0, :, 1, 5].float(),
+                               value * torch.sign(d["C"][0, :, 1, 3].float()))
+        assert float(hb[0, 1, 5, 3]) == value
+
+
 @pytest.mark.parametrize("L", [100, 256, 513, 2600])
 @pytest.mark.parametrize("disc", ["zoh", "euler"])
 @pytest.mark.parametrize("with_d", [False, True])

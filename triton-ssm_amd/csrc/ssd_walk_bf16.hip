@@ -35,6 +35,11 @@
 // B=1 L=65536 H=8: 119.8 us a call (before 139 - 144).  16 channels a wave measured
 // 115 - 129 us on the first shape, 12 waves a workgroup 118 (spills).
 //
+// x that is not finite is rare and kept apart: the wave that finds some in its
+// block (a dot product with zero of the loaded registers, 8 instructions) takes it
+// through products of its own, each output step over its own past, so that steps
+// before it stay as they are (88.5 us without, 88.1 with).
+//
 // The hi/lo operands keep 16 bits, which y's rounding hides and the fp32 final
 // state does not: 2.2e-6 of float64 on it, where fp32 products give 1e-7.  So bf16
 // at other head dims and state sizes, whose state is formed in fp32 throughout, is
@@ -83,6 +88,49 @@ __device__ inline void split4(const float* v, uint2& hi, uint2& lo) {
   lo.y = pk_bf16(v[2] - bf16_lo(hi.y), v[3] - bf16_hi(hi.y));
 }
 
+// Whether any of a block's x is not finite (uniform), from the registers it was
+// loaded into: x . 0 is zero or NaN.
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+template <typename Regs>
+__device__ inline bool any_not_finite(const Regs& x) {
+  const bf16x2_t zero = {};
+  float z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (const u32x4 v : x.v)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      z[k] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, (uint32_t)v[k]), zero,
+                                             z[k], false);
+  return __ballot((z[0] + z[1]) + (z[2] + z[3]) != 0.0f) != 0;
+}
+// x split into its finite values, which stay, and the others, which are moved to
+// xb (zero elsewhere): a product with zero weights, of steps before them, must
+// not meet them.
+template <int PB>
+__device__ inline void take_not_finite(s16x4_t (&xc)[2][PB], s16x4_t (&xb)[2][PB]) {
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int q = 0; q < PB; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const short v = xc[a][q][r];
+        const bool f = (v & 0x7f80) != 0x7f80;
+        xb[a][q][r] = f ? (short)0 : v;
+        xc[a][q][r] = f ? v : (short)0;
+      }
+}
+// x of rows r0 .. r0 + 3, zero after row `last`.
+__device__ inline s16x4_t past_only(s16x4_t x, int r0, int last) {
+  s16x4_t o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = r0 + r <= last ? x[r] : (short)0;
+  return o;
+}
+__device__ inline mfma_acc mfma16(s16x4_t x, uint2 m, mfma_acc acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(x, as_s16x4(m), acc, 0, 0, 0);
+}
+
 // One block's step quantities: lane l stands for step l % 32.  The log2 decays
 // are summed in fp32 over 16 steps at most.
 struct W16Steps {
@@ -107,9 +155,18 @@ __device__ inline W16Steps w16_steps(float d, float a2, bool zoh) {
   return o;
 }
 
+template <int PB>
+__device__ inline void zero_state(mfma_acc (&H)[NB][PB]) {
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int q = 0; q < PB; ++q) H[i][q] = mfma_acc{0.0f, 0.0f, 0.0f, 0.0f};
+}
+
 // H^T += sum_s w_s B_s x_s^T over the block's 32 steps: w the LDS weights,
-// xc the x columns read_cols gave for (half a, channel block q).
-template <typename In, int PB>
+// xc the x columns read_cols gave for (half a, channel block q).  HIGH: the high
+// parts of w x alone (x not finite, whose low parts would be inf - inf).
+template <typename In, int PB, bool HIGH = false>
 __device__ inline void w16_update(mfma_acc (&H)[NB][PB], const char* lds, const float* w,
                                   const s16x4_t (&xc)[2][PB], int c, int j) {
   bf16x8_t xh[PB], xl[PB];
@@ -137,7 +194,8 @@ __device__ inline void w16_update(mfma_acc (&H)[NB][PB], const char* lds, const 
 #pragma unroll
     for (int q = 0; q < PB; ++q) {
       H[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bt, xh[q], H[i][q], 0, 0, 0);
-      H[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bt, xl[q], H[i][q], 0, 0, 0);
+      if constexpr (!HIGH)
+        H[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bt, xl[q], H[i][q], 0, 0, 0);
     }
   }
 }
@@ -167,12 +225,10 @@ ssd_walk16_state_kernel(SsdArgs a, uint32_t npg, uint32_t nsub, uint32_t segb, i
   in.load(g1, at((int)segb - 2));
   const float a2 = -expf(a.A_log[u.h]) * kLog2e;
   mfma_acc H[NB][PB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i)
-#pragma unroll
-    for (int q = 0; q < PB; ++q) H[i][q] = mfma_acc{0.0f, 0.0f, 0.0f, 0.0f};
+  zero_state(H);
   float lsum = 0.0f;  // log2 decay of the blocks already taken (the later ones)
   auto step = [&](typename In::Regs& g, int kb) {
+    const bool bad = any_not_finite(g.x);
     const float d = in.stage(g, lds, at(kb));
     in.load(g, at(kb - 2));
     const W16Steps s = w16_steps(d, a2, zoh != 0);
@@ -185,6 +241,11 @@ ssd_walk16_state_kernel(SsdArgs a, uint32_t npg, uint32_t nsub, uint32_t segb, i
 #pragma unroll
       for (int q = 0; q < PB; ++q)
         xc[h][q] = read_cols<typename In::TX>(lds + In::kX, h, 16 * q, c, j);
+    if (bad) {
+      s16x4_t xb[2][PB];
+      take_not_finite(xc, xb);
+      w16_update<In, PB, true>(H, lds, w, xb, c, j);
+    }
     w16_update<In, PB>(H, lds, w, xc, c, j);
     lsum += s.tot0 + s.tot1;
     return exp2_fast(lsum) != 0.0f;  // uniform; at 0 every earlier weight is zero too
@@ -339,6 +400,7 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
   W16Steps s = weights(live_dt(in_flight.dt, t0), 0);
   int buf = 0;
   for (int64_t tb = blk0 * kW16Q; tb < t_end; tb += kSuper, t0 += kSuper, buf ^= 1) {
+    const bool bad = any_not_finite(in_flight.x);
     in.stage(in_flight, lds, t0);
     const W16Weights& sc = s_sc[wv][buf];
     const bool fac = s.tot0 >= -240.0f && s.tot1 >= -240.0f;
@@ -349,10 +411,7 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
 #pragma unroll
       for (int q = 0; q < PB; ++q) xc[h][q] = read_cols<TX>(lds + In::kX, h, 16 * q, c, j);
     mfma_acc H[NB][PB];
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int q = 0; q < PB; ++q) H[i][q] = mfma_acc{0.0f, 0.0f, 0.0f, 0.0f};
+    zero_state(H);
     w16_update<In, PB>(H, lds, sc.wu, xc, c, j);
     // the next block's loads, a part at a time: eight waves issuing all of
     // theirs at once wait on each other
@@ -383,6 +442,13 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
         for (int q = 0; q < PB; ++q)
           xd[t][q] = *reinterpret_cast<const uint2*>(lds + In::kX + (16 * t + c) * TX::kStride +
                                                      (16 * q + 4 * j) * 2);
+    }
+    s16x4_t xb[2][PB];
+    if (bad) {  // the share again (a branch before the update cost 1.7 us of 88)
+      take_not_finite(xc, xb);
+      zero_state(H);
+      w16_update<In, PB, true>(H, lds, sc.wu, xb, c, j);
+      w16_update<In, PB>(H, lds, sc.wu, xc, c, j);
     }
     wave_lds_order();
 #pragma unroll
@@ -467,14 +533,30 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
         y[0][q][r] *= z0;
         y[1][q][r] *= dec0;
       }
-      y[1][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xc[0][q], as_s16x4(h01), y[1][q], 0, 0, 0);
-      y[1][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xc[0][q], as_s16x4(l01), y[1][q], 0, 0, 0);
-      y[0][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xc[0][q], as_s16x4(h00), y[0][q], 0, 0, 0);
-      y[0][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xc[0][q], as_s16x4(l00), y[0][q], 0, 0, 0);
+      y[1][q] = mfma16(xc[0][q], h01, y[1][q]);
+      y[1][q] = mfma16(xc[0][q], l01, y[1][q]);
+      y[0][q] = mfma16(xc[0][q], h00, y[0][q]);
+      y[0][q] = mfma16(xc[0][q], l00, y[0][q]);
 #pragma unroll
       for (int r = 0; r < 4; ++r) y[1][q][r] *= z1;
-      y[1][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xc[1][q], as_s16x4(h11), y[1][q], 0, 0, 0);
-      y[1][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xc[1][q], as_s16x4(l11), y[1][q], 0, 0, 0);
+      y[1][q] = mfma16(xc[1][q], h11, y[1][q]);
+      y[1][q] = mfma16(xc[1][q], l11, y[1][q]);
+    }
+    if (bad) {  // each output step takes its own past of the x kept apart
+#pragma unroll
+      for (int q = 0; q < PB; ++q) {
+        y[1][q] = mfma16(xb[0][q], h01, y[1][q]);
+#pragma unroll 1
+        for (int tt = 0; tt < 16; ++tt) {
+          const mfma_acc p0 = mfma16(past_only(xb[0][q], 4 * j, tt), h00, y[0][q]);
+          const mfma_acc p1 = mfma16(past_only(xb[1][q], 4 * j, tt), h11, y[1][q]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            y[0][q][r] = c == tt ? p0[r] : y[0][q][r];
+            y[1][q][r] = c == tt ? p1[r] : y[1][q][r];
+          }
+        }
+      }
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
