@@ -115,6 +115,40 @@ def test_ssd_scan_bf16_walk(dev, B, L, H, P, N, chunk, decay, with_d):
     assert_close(hl, h_ref, 1e-3 if N == 64 and P % 16 == 0 else 2e-6, "bf16 walk h_last")
 
 
+@pytest.mark.parametrize("total", [-120, -127, -129, -160, -205, -220, -238, -250])
+@pytest.mark.parametrize("step", [1e-2, 1e-4])
+def test_ssd_scan_bf16_short_steps_before_a_gap(dev, total, step):
+    """15 short steps, then a gap that decays by 2^total: the outputs before the gap
+    are small beside those after it and still right on their own norm (the output's
+    bf16 rounding, 2^-9)."""
+    from tssm import ssd_scan_forward
+    d = _ssd_inputs(dev, 1, 64, 2, 64, 64, torch.bfloat16, seed=5, heavy=False)
+    d["A_log"].zero_()
+    d["dt"].fill_(step)
+    d["dt"][:, 15::16] = -total * np.log(2.0) - 15 * step
+    args = (d["x"], d["dt"], d["A_log"], d["B"], d["C"])
+    y, hl = ssd_scan_forward(*args, return_state=True)
+    y_ref, h_ref = O.ssd_scan(*args)
+    assert_close(y[:, :15], y_ref[:, :15], 4e-3, "before the gap")
+    assert_close(y, y_ref, 4e-3, "y")
+    assert_close(hl, h_ref, 1e-3, "h_last")
+
+
+@pytest.mark.parametrize("log2_decay", [6.0, 7.9, 8.1, 12.0, 14.5, 15.5])
+def test_ssd_scan_bf16_large_values(dev, log2_decay):
+    """Every step decays alike, B.C of a few thousand, Euler steps of 10 to 30: no
+    weight overflows on its way (the same bar as the other rows)."""
+    from tssm import ssd_scan_forward
+    d = _ssd_inputs(dev, 1, 96, 2, 64, 64, torch.bfloat16, seed=6, heavy=False)
+    d["A_log"].fill_(float(np.log(0.5)))
+    d["dt"].fill_(log2_decay * float(np.log(2.0)) / 0.5)
+    args = (d["x"], d["dt"], d["A_log"], d["B"] * 30, d["C"] * 30)
+    y, hl = ssd_scan_forward(*args, disc="euler", return_state=True)
+    y_ref, h_ref = O.ssd_scan(*args, disc="euler")
+    assert_close(y, y_ref, 4e-3, "y")
+    assert_close(hl, h_ref, 1e-3, "h_last")
+
+
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 @pytest.mark.parametrize("L,s", [(300, 151), (300, 15), (300, 32), (2000, 1111)])
 @pytest.mark.parametrize("P,N", [(64, 64), (16, 64), (24, 64), (32, 32)])

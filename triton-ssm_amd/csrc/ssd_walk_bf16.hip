@@ -15,9 +15,9 @@
 //   y_t (half 1) = u_t (2^(tot1/2) (2^tot0 H.C_t + sum_{half 0} (B_s.C_t) w_s x_s)
 //                       + sum_{s <= t} (B_s.C_t) v_s x_s)
 //   H' = 2^(tot0 + tot1) H + sum_s w_s 2^(tot of the later half) x_s B_s
-// Every factor stays within 2^+-120 while a half decays by at most 2^-240;
-// a block with a half beyond that takes its diagonal weights element by
-// element.  x, B and C enter the products exactly; operands formed in fp32
+// Every factor stays within 2^+-64 while a half decays by at most 2^-128
+// (kW16Factored); a block with a half beyond that takes its diagonal weights
+// element by element.  x, B and C enter the products exactly; operands formed in fp32
 // (weighted Gram blocks, weighted x, the state) are split into bf16 hi + lo
 // and multiplied twice, as in the other bf16 kernels.
 //
@@ -56,6 +56,14 @@ constexpr int NB = 4;      // column tiles of 16: N = 64
 // itself; more take the prefix pass.  Folding reads eight states where decays
 // forget and 15 rounds of eight at worst, the prefix pass 10-18 us either way.
 constexpr int64_t kW16Fold = 128;
+
+// Largest log2 decay of a half whose diagonal weights are formed as u_t v_s.  A
+// weighted Gram value B_s.C_t v_s may be 2^+-64 off its final size, is split into
+// bf16 hi and lo and summed with x: it must neither reach 2^128 (with 2^+-120 a half
+// of 2^-232 gave inf from B.C of a few hundred) nor lose its lo part, 2^-16 of it, at
+// 2^-126 (with 2^+-120 steps of 1e-4 before a long gap were off by their own size).
+// B=8 L=4096 H=16 P=N=64: 87.9 us with 2^+-120, 88.4 with 2^+-64.
+constexpr float kW16Factored = -128.0f;
 
 typedef __attribute__((address_space(3))) s16x4_t* lds_s16x4;
 
@@ -382,7 +390,7 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
   }
   auto weights = [&](float d, int b) {
     const W16Steps s = w16_steps(d, a2, zoh != 0);
-    const bool fac = s.tot0 >= -240.0f && s.tot1 >= -240.0f;  // uniform in the wave
+    const bool fac = s.tot0 >= kW16Factored && s.tot1 >= kW16Factored;  // uniform in the wave
     W16Weights& k = s_sc[wv][b];
     if (lane < kW16Q) {
       const float tot = lane < 16 ? s.tot0 : s.tot1;
@@ -403,7 +411,7 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
     const bool bad = any_not_finite(in_flight.x);
     in.stage(in_flight, lds, t0);
     const W16Weights& sc = s_sc[wv][buf];
-    const bool fac = s.tot0 >= -240.0f && s.tot1 >= -240.0f;
+    const bool fac = s.tot0 >= kW16Factored && s.tot1 >= kW16Factored;
     // every operand of the block into registers, and what needs no state
     s16x4_t xc[2][PB];
 #pragma unroll
