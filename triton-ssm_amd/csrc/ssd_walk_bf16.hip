@@ -140,9 +140,14 @@ __device__ inline mfma_acc mfma16(s16x4_t x, uint2 m, mfma_acc acc) {
 }
 
 // One block's step quantities: lane l stands for step l % 32.  The log2 decays
-// are summed in fp32 over 16 steps at most.
+// are summed in fp32 over 16 steps at most, forwards for the outputs and, for the
+// state, backwards: 2^(tot - cum) after a long gap would keep the gap's rounding
+// (1e-4 on the state after steps of 700; with `after` 3e-6).  kW16Floor: one step's
+// decay is 0 either way, and what follows it keeps its bits.
+constexpr float kW16Floor = -256.0f;
 struct W16Steps {
   float cum, tot0, tot1;  // within the step's half; the halves' sums (uniform)
+  float after;            // of the half's steps after this one
   float coef;
 };
 __device__ inline float lane_f32(float v, int lane) {
@@ -152,7 +157,13 @@ __device__ inline W16Steps w16_steps(float d, float a2, bool zoh) {
   W16Steps o;
   const float y = d * a2;
   o.coef = zoh ? phi1_from_exp(y * 0.6931471805599453f, exp2_fast(y)) * d : d;
-  float l = y < (float)kWalkFloor ? (float)kWalkFloor : y;
+  float l = y < kW16Floor ? kW16Floor : y;
+  float r = dpp_in<0x101, 0xf>(l);  // row_shl:1
+  r += dpp_in<0x101, 0xf>(r);
+  r += dpp_in<0x102, 0xf>(r);
+  r += dpp_in<0x104, 0xf>(r);
+  r += dpp_in<0x108, 0xf>(r);
+  o.after = r;
   l += dpp_in<0x111, 0xf>(l);
   l += dpp_in<0x112, 0xf>(l);
   l += dpp_in<0x114, 0xf>(l);
@@ -240,8 +251,8 @@ ssd_walk16_state_kernel(SsdArgs a, uint32_t npg, uint32_t nsub, uint32_t segb, i
     const float d = in.stage(g, lds, at(kb));
     in.load(g, at(kb - 2));
     const W16Steps s = w16_steps(d, a2, zoh != 0);
-    const float after = lsum + ((lane & 16) ? s.tot1 : s.tot0 + s.tot1);
-    if (lane < kW16Q) w[lane] = exp2_fast(after - s.cum) * s.coef;
+    const float later = (lane & 16) ? lsum : lsum + s.tot1;
+    if (lane < kW16Q) w[lane] = exp2_fast(later + s.after) * s.coef;
     wave_lds_order();
     s16x4_t xc[2][PB];
 #pragma unroll
@@ -394,12 +405,12 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
     W16Weights& k = s_sc[wv][b];
     if (lane < kW16Q) {
       const float tot = lane < 16 ? s.tot0 : s.tot1;
-      const float wl = exp2_fast(tot - s.cum) * s.coef;
+      const float wl = exp2_fast(s.after) * s.coef;
       k.u[lane] = exp2_fast(fac ? s.cum - 0.5f * tot : s.cum);
       k.v[lane] = fac ? exp2_fast(0.5f * tot - s.cum) * s.coef : s.coef;
       k.w[lane] = wl;
       // to the block's end, for the state
-      k.wu[lane] = lane < 16 ? exp2_fast(s.tot0 + s.tot1 - s.cum) * s.coef : wl;
+      k.wu[lane] = lane < 16 ? exp2_fast(s.tot1 + s.after) * s.coef : wl;
       k.cum[lane] = s.cum;
     }
     if (lane == 0) s_dec[b][wv] = exp2_fast(s.tot0 + s.tot1);
