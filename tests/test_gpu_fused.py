@@ -95,6 +95,9 @@ def test_ssd_scan_walk(dev, dtype, B, L, H, P, N, chunk, form):
     (1, 700, 2, 24, 64, 256, "gaps", True),
     (1, 700, 2, 64, 64, 256, "gaps", True),
     (1, 6000, 1, 32, 64, 64, "gaps", False),
+    (1, 33024, 1, 32, 64, 256, "slow", True),      # 129 segments: the prefix pass
+    (1, 66000, 1, 16, 64, 256, "still", True),     # as many of two super-blocks, the last ragged
+    (1, 32768, 1, 16, 64, 256, "still", True),     # 128: the last that the output pass folds, all
 ])
 def test_ssd_scan_bf16_walk(dev, B, L, H, P, N, chunk, decay, with_d):
     """bf16 with N = 64 or 32 at the edges of the walks' blocks, super-blocks,
@@ -105,7 +108,8 @@ def test_ssd_scan_bf16_walk(dev, B, L, H, P, N, chunk, decay, with_d):
     as in test_ssd_scan_walk)."""
     from tssm import ssd_scan_forward
     d = _ssd_inputs(dev, B, L, H, P, N, torch.bfloat16, seed=L + P + N, heavy=False)
-    d["dt"] = d["dt"] * {"plain": 1.0, "fast": 40.0, "slow": 0.003, "gaps": 0.01}[decay]
+    d["dt"] = d["dt"] * {"plain": 1.0, "fast": 40.0, "slow": 0.003, "still": 1e-5,
+                          "gaps": 0.01}[decay]
     if decay == "gaps":
         d["dt"][:, ::37] = 700.0
     h0 = torch.randn(B, H, P, N, device=dev)
@@ -213,7 +217,7 @@ def test_ssd_scan_matrix_core_path(dev, L, disc, with_d):
 def test_ssd_scan_time_broadcast_b(dev):
     """bf16 P=64 N=16 with B broadcast over time (row stride 0): the matrix-core
     tile passes need every row stride to cover a row, so this layout runs the
-    generic passes, against the same oracle."""
+    fp32-product walk, against the same oracle."""
     from tssm import ssd_scan_forward
     d = _ssd_inputs(dev, 2, 700, 3, 64, 16, torch.bfloat16, seed=77, heavy=True)
     Bb = d["B"][:, :1].expand(-1, 700, -1, -1)
@@ -229,10 +233,10 @@ def test_ssd_scan_time_broadcast_b(dev):
 @pytest.mark.parametrize("disc", ["zoh", "euler"])
 @pytest.mark.parametrize("with_d", [False, True])
 def test_ssd_scan_n64_matrix_core_path(dev, Bsz, L, H, P, disc, with_d):
-    """bf16 with N = 64 runs one matrix-core pass per (row, 16-channel block):
-    ragged blocks of 64 steps, 1-4 channel blocks per row, row counts that are
-    and are not multiples of 8 (the two block mappings), skip term, nonzero h0
-    and the final state.  Same bar as the other matrix-core path."""
+    """bf16 with N = 64 and P a multiple of 16 on the bf16 walk: ragged blocks of 32
+    steps and super-blocks of 256, one or two blocks of 32 channels a row (P = 16:
+    one of 16), (batch, segment) counts that are no multiple of 8, skip term, nonzero
+    h0 and the final state.  Same bar as the other matrix-core path."""
     from tssm import ssd_scan_forward
     d = _ssd_inputs(dev, Bsz, L, H, P, 64, torch.bfloat16, seed=L + P + with_d, heavy=True)
     h0 = torch.randn(Bsz, H, P, 64, device=dev)
@@ -247,7 +251,7 @@ def test_ssd_scan_n64_matrix_core_path(dev, Bsz, L, H, P, disc, with_d):
 
 @pytest.mark.parametrize("cut", [128, 200, 1])
 def test_ssd_scan_n64_split_resume(dev, cut):
-    """bf16 N = 64 on the one-pass matrix-core kernel: a run split at `cut`
+    """bf16 N = 64 on the bf16 walk: a run split at `cut`
     (the second half starting at an offset view of the same tensors) and
     resumed from the first half's final state reproduces the whole run."""
     from tssm import ssd_scan_forward
@@ -262,17 +266,17 @@ def test_ssd_scan_n64_split_resume(dev, cut):
 
 
 @pytest.mark.parametrize("Bsz,L,H,P,decay", [
-    (1, 5000, 2, 64, "slow"),    # 2 rows x 2 channel blocks: 20 segments of 256 steps, ragged end
+    (1, 5000, 2, 64, "slow"),    # 2 rows x 2 channel blocks: 10 segments of 512 steps, ragged end
     (1, 5000, 2, 64, "heavy"),
-    (1, 3001, 3, 48, "slow"),    # 3 rows (not a multiple of 8), 3 blocks of 16 channels
-    (2, 2000, 1, 16, "slow"),    # one 16-channel block: the step halves of pass 1 added
-    (1, 4000, 8, 32, "slow"),    # 8 rows (XCD mapping), one 32-channel block per row
+    (1, 3001, 3, 48, "slow"),    # 6 segments; the second channel block of a row half empty
+    (2, 2000, 1, 16, "slow"),    # one 16-channel block a row, 4 segments
+    (1, 4000, 8, 32, "slow"),    # 8 segments (XCD mapping), one 32-channel block per row
 ])
 @pytest.mark.parametrize("disc", ["zoh", "euler"])
 def test_ssd_scan_n64_segments(dev, Bsz, L, H, P, decay, disc):
-    """bf16 N = 64 with too few (row, channel block) units to fill the chip:
-    the one-pass kernel runs time segments (pass 1 segment end states, the
-    prefix pass over segments, pass 3 outputs from each entry state).  Slow
+    """bf16 N = 64 with too few (row, channel block) units to fill the chip: the
+    bf16 walk cuts the sequence into time segments (pass 1 forms the end states of
+    the earlier sub-segments, the output pass folds them into its entry state).  Slow
     decays carry the state across every segment; h0, skip term and the final
     state against the float64 oracle."""
     from tssm import ssd_scan_forward
@@ -293,10 +297,10 @@ def test_ssd_scan_n64_segments(dev, Bsz, L, H, P, decay, disc):
 
 @pytest.mark.parametrize("chunk", [64, 1024])
 def test_ssd_scan_n64_segments_chunk_slots(dev, chunk):
-    """The segment count is bounded by the workspace's chunk slots: with
-    1024-step chunks (L=5000: 5 slots) there are fewer segments and one
-    sub-segment per segment in pass 1; with 64-step chunks more sub-segments
-    fit.  Slow decays, h0, skip term, against the float64 oracle."""
+    """Segments and sub-segments are bounded by the workspace's chunk slots: with
+    1024-step chunks (L=5000: room for 9 states) 7 segments, one sub-segment each;
+    with 64-step chunks 10 of two sub-segments.  Slow decays, h0, skip term,
+    against the float64 oracle."""
     from tssm import ssd_scan_forward
     Bsz, L, H, P = 1, 5000, 2, 64
     d = _ssd_inputs(dev, Bsz, L, H, P, 64, torch.bfloat16, seed=chunk, heavy=True)
@@ -314,7 +318,7 @@ def test_ssd_scan_n64_segments_chunk_slots(dev, chunk):
 
 def test_ssd_scan_n64_long_sequence(dev):
     """B=1 L=65536 H=8 P=N=64 bf16, log-normal dt: 16 (row, channel block)
-    units, so the one-pass kernel runs 16 segments of 4096 steps.  Heads 0
+    units, so the walk runs 16 segments of 4096 steps.  Heads 0
     and 7 against the float64 oracle over every step, every head against the
     oracle's fp32 C restatement, and split/resume at L/2."""
     import tssm
