@@ -948,7 +948,7 @@ extern "C" int tssm_ssd_scan(int dtype, int disc, const void* x, const float* dt
   const hipStream_t s = as_stream(stream);
   const bool has_d = D != nullptr;
   // bf16 at P = 64, N = 16 with 256-step tiles: matrix-core passes (other
-  // row strides take the generic passes)
+  // row strides take the fp32-product walk)
   int64_t wseg = ssd_wave_seg(rows, nchunks);
   if (wseg > 1 && !ssd_wave_ok(a, wseg * kMq)) wseg = 1;  // row strides too long for a segment
   if (dtype == TSSM_BF16 && P == kMp && N == kMn && tc == kMq && ssd_wave_ok(a, wseg * kMq)) {

@@ -1,5 +1,5 @@
 // Shapes and matrix-core helpers shared by the SSD translation units
-// (ssd.hip: generic passes, N = 16 tile passes, one-launch kernel, streaming
+// (ssd.hip: N = 16 tile passes, one-launch kernel, streaming
 // step; ssd_walk.hip, ssd_walk_bf16.hip: every other form).
 #pragma once
 

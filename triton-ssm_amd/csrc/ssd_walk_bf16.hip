@@ -612,8 +612,11 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
 // all of them (B=1 L=65536 H=8 P=N=64, slow decays: 190 us with m = 1, 132 with
 // m = 8), and no more of them than the output pass folds itself (B=1 L=100000
 // H=1: 53 us with 389 and the prefix pass, 30 with 98; slow decays 59 and 53).
-// Segments of one super-block beat two where units are few: B=1 L=20000 H=1
-// 23.5 -> 19.8 us, slow decays 33.2 -> 29.6; L=700 pays, 15.8 -> 16.6.
+// The count is bounded first and the length then rounded up to whole super-blocks,
+// so that a segment is one super-block only where the blocks fill them: L=20000,
+// 625 blocks, gives 40 segments of two, where a bound of two super-blocks gives 27
+// of three (B=1 H=1 23.5 -> 19.8 us, slow decays 33.2 -> 29.6; L=700, two segments
+// instead of one, pays: 15.8 -> 16.6).
 constexpr int64_t kW16MinSuper = 1, kW16StateWaves = 2048, kW16MinSub = 8;
 template <int PB>
 int launch_walk16(int disc, hipStream_t s, SsdArgs a) {
