@@ -35,10 +35,10 @@
 // B=1 L=65536 H=8: 119.8 us a call (before 139 - 144).  16 channels a wave measured
 // 115 - 129 us on the first shape, 12 waves a workgroup 118 (spills).
 //
-// x that is not finite is rare and kept apart: the wave that finds some in its
-// block (a dot product with zero of the loaded registers, 8 instructions) takes it
-// through products of its own, each output step over its own past, so that steps
-// before it stay as they are (88.5 us without, 88.1 with).
+// x that is not finite is rare.  The wave that finds some in its block (a dot
+// product with zero of the loaded registers, 8 instructions) takes it through
+// products of its own, each output step over its own past, so that steps before it
+// stay as they are (88.5 us without, 88.4 with).  It makes its channel's state NaN.
 //
 // The hi/lo operands keep 16 bits, which y's rounding hides and the fp32 final
 // state does not: 2.2e-6 of float64 on it, where fp32 products give 1e-7.  So bf16
@@ -174,18 +174,9 @@ __device__ inline W16Steps w16_steps(float d, float a2, bool zoh) {
   return o;
 }
 
-template <int PB>
-__device__ inline void zero_state(mfma_acc (&H)[NB][PB]) {
-#pragma unroll
-  for (int i = 0; i < NB; ++i)
-#pragma unroll
-    for (int q = 0; q < PB; ++q) H[i][q] = mfma_acc{0.0f, 0.0f, 0.0f, 0.0f};
-}
-
 // H^T += sum_s w_s B_s x_s^T over the block's 32 steps: w the LDS weights,
-// xc the x columns read_cols gave for (half a, channel block q).  HIGH: the high
-// parts of w x alone (x not finite, whose low parts would be inf - inf).
-template <typename In, int PB, bool HIGH = false>
+// xc the x columns read_cols gave for (half a, channel block q).
+template <typename In, int PB>
 __device__ inline void w16_update(mfma_acc (&H)[NB][PB], const char* lds, const float* w,
                                   const s16x4_t (&xc)[2][PB], int c, int j) {
   bf16x8_t xh[PB], xl[PB];
@@ -213,8 +204,7 @@ __device__ inline void w16_update(mfma_acc (&H)[NB][PB], const char* lds, const 
 #pragma unroll
     for (int q = 0; q < PB; ++q) {
       H[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bt, xh[q], H[i][q], 0, 0, 0);
-      if constexpr (!HIGH)
-        H[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bt, xl[q], H[i][q], 0, 0, 0);
+      H[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bt, xl[q], H[i][q], 0, 0, 0);
     }
   }
 }
@@ -244,10 +234,12 @@ ssd_walk16_state_kernel(SsdArgs a, uint32_t npg, uint32_t nsub, uint32_t segb, i
   in.load(g1, at((int)segb - 2));
   const float a2 = -expf(a.A_log[u.h]) * kLog2e;
   mfma_acc H[NB][PB];
-  zero_state(H);
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int q = 0; q < PB; ++q) H[i][q] = mfma_acc{0.0f, 0.0f, 0.0f, 0.0f};
   float lsum = 0.0f;  // log2 decay of the blocks already taken (the later ones)
   auto step = [&](typename In::Regs& g, int kb) {
-    const bool bad = any_not_finite(g.x);
     const float d = in.stage(g, lds, at(kb));
     in.load(g, at(kb - 2));
     const W16Steps s = w16_steps(d, a2, zoh != 0);
@@ -260,11 +252,6 @@ ssd_walk16_state_kernel(SsdArgs a, uint32_t npg, uint32_t nsub, uint32_t segb, i
 #pragma unroll
       for (int q = 0; q < PB; ++q)
         xc[h][q] = read_cols<typename In::TX>(lds + In::kX, h, 16 * q, c, j);
-    if (bad) {
-      s16x4_t xb[2][PB];
-      take_not_finite(xc, xb);
-      w16_update<In, PB, true>(H, lds, w, xb, c, j);
-    }
     w16_update<In, PB>(H, lds, w, xc, c, j);
     lsum += s.tot0 + s.tot1;
     return exp2_fast(lsum) != 0.0f;  // uniform; at 0 every earlier weight is zero too
@@ -430,7 +417,10 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
 #pragma unroll
       for (int q = 0; q < PB; ++q) xc[h][q] = read_cols<TX>(lds + In::kX, h, 16 * q, c, j);
     mfma_acc H[NB][PB];
-    zero_state(H);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int q = 0; q < PB; ++q) H[i][q] = mfma_acc{0.0f, 0.0f, 0.0f, 0.0f};
     w16_update<In, PB>(H, lds, sc.wu, xc, c, j);
     // the next block's loads, a part at a time: eight waves issuing all of
     // theirs at once wait on each other
@@ -463,12 +453,7 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
                                                      (16 * q + 4 * j) * 2);
     }
     s16x4_t xb[2][PB];
-    if (bad) {  // the share again (a branch before the update cost 1.7 us of 88)
-      take_not_finite(xc, xb);
-      zero_state(H);
-      w16_update<In, PB, true>(H, lds, sc.wu, xb, c, j);
-      w16_update<In, PB>(H, lds, sc.wu, xc, c, j);
-    }
+    if (__builtin_expect(bad, false)) take_not_finite(xc, xb);  // (the share has it already)
     wave_lds_order();
 #pragma unroll
     for (int q = 0; q < PB; ++q)
@@ -561,7 +546,7 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
       y[1][q] = mfma16(xc[1][q], h11, y[1][q]);
       y[1][q] = mfma16(xc[1][q], l11, y[1][q]);
     }
-    if (bad) {  // each output step takes its own past of the x kept apart
+    if (__builtin_expect(bad, false)) {  // each output step's own past of the x kept apart
 #pragma unroll
       for (int q = 0; q < PB; ++q) {
         y[1][q] = mfma16(xb[0][q], h01, y[1][q]);
