@@ -89,15 +89,19 @@ def test_ssd_scan_walk(dev, dtype, B, L, H, P, N, chunk, form):
     (1, 257, 2, 40, 64, 256, "fast", False),       # one step into the second super-block
     (2, 3000, 3, 64, 64, 256, "slow", True),       # segments, states folded
     (2, 3000, 3, 64, 32, 64, "plain", True),
-    (1, 9000, 1, 16, 64, 64, "slow", False),       # sub-segments of pass 1
+    (1, 9000, 1, 16, 64, 64, "slow", False),
+    (2, 8000, 8, 64, 64, 256, "slow", False),      # four sub-segments of pass 1 a segment
     (65, 300, 4, 64, 32, 256, "plain", False),     # more workgroups than CUs
     (1, 700, 2, 64, 32, 256, "gaps", True),        # long gaps between short steps
     (1, 700, 2, 24, 64, 256, "gaps", True),
     (1, 700, 2, 64, 64, 256, "gaps", True),
     (1, 6000, 1, 32, 64, 64, "gaps", False),
-    (1, 33024, 1, 32, 64, 256, "slow", True),      # 129 segments: the prefix pass
-    (1, 66000, 1, 16, 64, 256, "still", True),     # as many of two super-blocks, the last ragged
-    (1, 32768, 1, 16, 64, 256, "still", True),     # 128: the last that the output pass folds, all
+    (1, 700, 2, 32, 64, 256, "slow", True),        # three segments of one super-block
+    (1, 512, 2, 32, 64, 256, "slow", False),       # two super-blocks in one segment
+    (1, 32768, 1, 16, 64, 256, "still", True),     # 128 of one, all folded
+    (1, 65536, 1, 16, 64, 256, "still", False),    # 128 of two, the most that are folded
+    (1, 66000, 1, 16, 64, 256, "still", True),     # 129, the last ragged: the prefix pass
+    (1, 100000, 1, 32, 64, 256, "slow", True),     # 196
 ])
 def test_ssd_scan_bf16_walk(dev, B, L, H, P, N, chunk, decay, with_d):
     """bf16 with N = 64 or 32 at the edges of the walks' blocks, super-blocks,
@@ -267,11 +271,11 @@ def test_ssd_scan_n64_split_resume(dev, cut):
 
 
 @pytest.mark.parametrize("Bsz,L,H,P,decay", [
-    (1, 5000, 2, 64, "slow"),    # 2 rows x 2 channel blocks: 10 segments of 512 steps, ragged end
+    (1, 5000, 2, 64, "slow"),    # 2 rows x 2 channel blocks: 20 segments of 256 steps, ragged end
     (1, 5000, 2, 64, "heavy"),
-    (1, 3001, 3, 48, "slow"),    # 6 segments; the second channel block of a row half empty
-    (2, 2000, 1, 16, "slow"),    # one 16-channel block a row, 4 segments
-    (1, 4000, 8, 32, "slow"),    # 8 segments (XCD mapping), one 32-channel block per row
+    (1, 3001, 3, 48, "slow"),    # 12 segments; the second channel block of a row half empty
+    (2, 2000, 1, 16, "slow"),    # one 16-channel block a row, 8 segments
+    (1, 4000, 8, 32, "slow"),    # 16 segments (XCD mapping), one 32-channel block per row
 ])
 @pytest.mark.parametrize("disc", ["zoh", "euler"])
 def test_ssd_scan_n64_segments(dev, Bsz, L, H, P, decay, disc):
@@ -299,9 +303,9 @@ def test_ssd_scan_n64_segments(dev, Bsz, L, H, P, decay, disc):
 @pytest.mark.parametrize("chunk", [64, 1024])
 def test_ssd_scan_n64_segments_chunk_slots(dev, chunk):
     """Segments and sub-segments are bounded by the workspace's chunk slots: with
-    1024-step chunks (L=5000: room for 9 states) 7 segments, one sub-segment each;
-    with 64-step chunks 10 of two sub-segments.  Slow decays, h0, skip term,
-    against the float64 oracle."""
+    1024-step chunks (L=5000: room for 9 states) 7 segments of three super-blocks;
+    with 64-step chunks 20 of one.  Slow decays, h0, skip term, against the float64
+    oracle."""
     from tssm import ssd_scan_forward
     Bsz, L, H, P = 1, 5000, 2, 64
     d = _ssd_inputs(dev, Bsz, L, H, P, 64, torch.bfloat16, seed=chunk, heavy=True)

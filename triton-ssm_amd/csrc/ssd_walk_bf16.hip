@@ -590,19 +590,21 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
   }
 }
 
-// Time segments: as many as fill every CU once, each of at least kW16MinSuper
-// super-blocks (a segment costs pass 1 over its end, a launch, and its state twice
-// through memory).  Pass 1 takes a segment in m sub-segments of at least
-// kW16MinSub blocks, up to two of its waves a SIMD: with slow decays it walks
-// all of them (B=1 L=65536 H=8 P=N=64, slow decays: 190 us with m = 1, 132 with
-// m = 8), and no more of them than the output pass folds itself (B=1 L=100000
-// H=1: 53 us with 389 and the prefix pass, 30 with 98; slow decays 59 and 53).
-// The count is bounded first and the length then rounded up to whole super-blocks,
-// so that a segment is one super-block only where the blocks fill them: L=20000,
-// 625 blocks, gives 40 segments of two, where a bound of two super-blocks gives 27
-// of three (B=1 H=1 23.5 -> 19.8 us, slow decays 33.2 -> 29.6; L=700, two segments
-// instead of one, pays: 15.8 -> 16.6).
-constexpr int64_t kW16MinSuper = 1, kW16StateWaves = 2048, kW16MinSub = 8;
+// Time segments: as many as fill every CU once, each of at least one super-block,
+// and one only where two super-blocks hold the sequence (a segment costs pass 1 over
+// its end, a launch, and its state twice through memory: B=1 H=2 P=64 L=500 11.7 us
+// in one, 13.6 in two, 18.3 with slow decays; L=700 15.6 and 15.4 in one, 13.4 and
+// 18.5 in three).  Super-blocks are counted up: counted down they left segments of
+// two and half the CUs idle (L=2000 17.6 us, slow decays 22.1; with eight of one
+// 13.9 and 18.7).  No more than the output pass folds while two super-blocks each
+// suffice (B=1 H=1 P=32 L=40000 23.7 us with the prefix pass, slow decays 27.9;
+// folded 17.5 and 29.7); beyond, longer segments lose more than the prefix pass takes
+// (L=100000, slow decays: 49 us folded, 40).  Pass 1 takes a segment in m sub-segments of at least kW16MinSub
+// blocks, up to two of its waves a SIMD: with slow decays it walks all of them (B=1
+// L=65536 H=8 P=N=64, slow decays: 190 us with m = 1, 132 with m = 8), and no more of
+// them than the output pass folds itself (B=1 L=100000 H=1: 53 us with 389 and the
+// prefix pass, 30 with 98; slow decays 59 and 53).
+constexpr int64_t kW16StateWaves = 2048, kW16MinSub = 8;
 template <int PB>
 int launch_walk16(int disc, hipStream_t s, SsdArgs a) {
   const int64_t PN = (int64_t)a.P * (16 * NB), nblk = cdiv64(a.L, kW16Q), npg = cdiv64(a.P, 16 * PB);
@@ -610,10 +612,11 @@ int launch_walk16(int disc, hipStream_t s, SsdArgs a) {
   // a slot takes one state and one decay of the workspace, which holds two
   // states and a decay per chunk
   const int64_t cap = (int64_t)a.nchunks * (2 * PN + 1) / (PN + 1);
-  const int64_t by_len = nblk / (kW16MinSuper * kW16Waves);
+  const int64_t by_len = nblk <= 2 * kW16Waves ? 1 : cdiv64(nblk, kW16Waves);
   int64_t nseg = 256 / units;
   nseg = nseg < cap ? nseg : cap;
   nseg = nseg < by_len ? nseg : by_len;
+  if (nseg > kW16Fold && nblk <= 2 * kW16Waves * kW16Fold) nseg = kW16Fold;
   if (nseg < 1) nseg = 1;
   // whole super-blocks
   const int64_t segb = cdiv64(cdiv64(nblk, nseg), kW16Waves) * kW16Waves;
