@@ -28,12 +28,11 @@
 // are read from row-major LDS by ds_read_b64_tr_b16.
 //
 // Bound by the chain of dependent phases with one workgroup (two waves a SIMD) on a
-// CU, not by HBM: B=8 L=4096 H=16 P=N=64 takes 86.9 us with 271 MB moved (the one-pass
-// kernel it replaced: 101.1), about 53 at a copy's rate.  A super-block of 8 x 32
-// steps cost a wave 10,200 cycles while the decays were summed in fp64 (90 us), no
-// phase over a fifth of them.
-// B=1 L=65536 H=8: 119.8 us a call (before 139 - 144).  16 channels a wave measured
-// 115 - 129 us on the first shape, 12 waves a workgroup 118 (spills).
+// CU, not by HBM: B=8 L=4096 H=16 P=N=64 takes 88.4 us with 271 MB moved (the one-pass
+// kernel it replaced: 100.8), about 53 at a copy's rate.  A super-block of 8 x 32
+// steps costs a wave 10,350 cycles, no phase over a fifth of them.
+// B=1 L=65536 H=8: 119.8 - 123.8 us a call by box (before 139 - 144).  16 channels a
+// wave measured 115 - 129 us on the first shape, 12 waves a workgroup 118 (spills).
 //
 // x that is not finite is rare.  The wave that finds some in its block (a dot
 // product with zero of the loaded registers, 8 instructions) takes it through
