@@ -17,9 +17,10 @@
 //   H' = 2^(tot0 + tot1) H + sum_s w_s 2^(tot of the later half) x_s B_s
 // Every factor stays within 2^+-64 while a half decays by at most 2^-128
 // (kW16Factored); a block with a half beyond that takes its diagonal weights
-// element by element.  x, B and C enter the products exactly; operands formed in fp32
-// (weighted Gram blocks, weighted x, the state) are split into bf16 hi + lo
-// and multiplied twice, as in the other bf16 kernels.
+// element by element.  w comes from sums taken backwards (W16Steps).  x, B and C
+// enter the products exactly; operands formed in fp32 (weighted Gram blocks,
+// weighted x, the state) are split into bf16 hi + lo and multiplied twice, as in
+// the other bf16 kernels.
 //
 // No operand is transposed by instructions: Gram blocks and the state come out
 // of one product in the layout the next one takes (the order of k is free, so
@@ -53,7 +54,7 @@ constexpr int kW16Q = 32;  // steps per block
 constexpr int NB = 4;      // column tiles of 16: N = 64
 // Most sub-segments whose end states the output pass folds into entry states
 // itself; more take the prefix pass.  Folding reads eight states where decays
-// forget and 15 rounds of eight at worst, the prefix pass 10-18 us either way.
+// forget and 16 rounds of eight at worst, the prefix pass 10-18 us either way.
 constexpr int64_t kW16Fold = 128;
 
 // Largest log2 decay of a half whose diagonal weights are formed as u_t v_s.  A
@@ -598,15 +599,17 @@ ssd_walk16_out_kernel(SsdArgs a, uint32_t npg, uint32_t nseg, uint32_t segb, uin
 // 13.9 and 18.7).  No more than the output pass folds while two super-blocks each
 // suffice (B=1 H=1 P=32 L=40000 23.7 us with the prefix pass, slow decays 27.9;
 // folded 17.5 and 29.7); beyond, longer segments lose more than the prefix pass takes
-// (L=100000, slow decays: 49 us folded, 40).  Pass 1 takes a segment in m sub-segments of at least kW16MinSub
-// blocks, up to two of its waves a SIMD: with slow decays it walks all of them (B=1
-// L=65536 H=8 P=N=64, slow decays: 190 us with m = 1, 132 with m = 8), and no more of
-// them than the output pass folds itself (B=1 L=100000 H=1: 53 us with 389 and the
-// prefix pass, 30 with 98; slow decays 59 and 53).
+// (L=100000, slow decays: 49 us folded, 40).
+// Pass 1 takes a segment in m sub-segments of at least kW16MinSub blocks, up to two of
+// its waves a SIMD: with slow decays it walks all of them (B=1 L=65536 H=8 P=N=64, slow
+// decays: 190 us with m = 1, 132 with m = 8), and no more of them than the output pass
+// folds itself (B=1 L=100000 H=1: 53 us with 389 and the prefix pass, 30 with 98; slow
+// decays 59 and 53).
 constexpr int64_t kW16StateWaves = 2048, kW16MinSub = 8;
 template <int PB>
 int launch_walk16(int disc, hipStream_t s, SsdArgs a) {
-  const int64_t PN = (int64_t)a.P * (16 * NB), nblk = cdiv64(a.L, kW16Q), npg = cdiv64(a.P, 16 * PB);
+  const int64_t PN = (int64_t)a.P * (16 * NB), nblk = cdiv64(a.L, kW16Q);
+  const int64_t npg = cdiv64(a.P, 16 * PB);
   const int64_t units = (int64_t)a.rows * npg;
   // a slot takes one state and one decay of the workspace, which holds two
   // states and a decay per chunk
